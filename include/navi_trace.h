@@ -59,7 +59,7 @@ typedef struct navi_launch_info {
     uint32_t queue;        /* NAVI_QUEUE_* kind of work-queue pair the launch used */
     int32_t pair;          /* index of that pair in the device's table, -1 for none / scratch */
     uint32_t fast_planes;  /* split-plane depth staged by trace_fast_kernel (0: not enqueued) */
-    uint32_t planes;       /* split-plane depth staged by trace_relaid_kernel (0: none) */
+    uint32_t planes;       /* split-plane depth staged by trace_relaid_kernel or trace_quad_kernel (0: none) */
     uint32_t staged;       /* 1 when finished rays are staged per tile in LDS */
     uint32_t waves;        /* waves of the tracing grid (trace_fast_kernel's when enqueued) */
     uint64_t n_rays;
@@ -73,8 +73,10 @@ typedef struct navi_launch_info {
 #define NAVI_KERNEL_FAST_WIDE 2u    /* ... in 1024-thread workgroups (two per CU) */
 #define NAVI_KERNEL_COMBINED 4u     /* trace_relaid_kernel (both marches, seven waves per SIMD) */
 #define NAVI_KERNEL_RAW 8u          /* the word-layout kernel (navi_cast_rays, navi_cast_rays_multi) */
+#define NAVI_KERNEL_QUAD 16u        /* with COMBINED: trace_quad_kernel instead (both marches, four lanes per ray) */
 /* navi_launch_info.queue */
-#define NAVI_QUEUE_NONE 0u     /* no pair: static schedule, trace_fast_kernel not enqueued */
+#define NAVI_QUEUE_NONE 0u     /* no pair: trace_quad_kernel, which needs none, or a static schedule
+                                  without trace_fast_kernel */
 #define NAVI_QUEUE_STREAM 1u   /* the stream's pair */
 #define NAVI_QUEUE_CAPTURE 2u  /* a pair of the graph being captured */
 #define NAVI_QUEUE_LEASE 3u    /* a reserve pair leased for this launch */
@@ -351,8 +353,9 @@ int navi_trace_relaid_ex(const navi_relaid_launch* launch, void* stream);
  * Launch shape of the record-layout tracer (no reference counterpart: a tuning
  * knob of this library). Launches of at least `n_rays` rays whose scenes'
  * split planes fit two levels below the cell tables in 80 KiB of LDS run in
- * 1024-thread workgroups (two per CU); smaller launches, whose few workgroups
- * then spread over more CUs, in 256-thread ones. Results are identical either
+ * 1024-thread workgroups (two per CU), a lane per ray; smaller launches below
+ * 2^19 rays run with four lanes per ray (trace_quad_kernel), smaller launches
+ * of 2^19 rays and more in 256-thread workgroups. Results are identical either
  * way. Process-wide, thread-safe; takes effect from the next launch. Returns
  * the previous value (default 2^19).
  */

@@ -149,7 +149,7 @@ _lib.navi_last_launch.restype = ctypes.c_int
 _lib.navi_last_launch.argtypes = [ctypes.POINTER(LaunchInfo)]
 
 # navi_launch_info bits and kinds (include/navi_trace.h)
-KERNEL_FAST, KERNEL_FAST_WIDE, KERNEL_COMBINED, KERNEL_RAW = 1, 2, 4, 8
+KERNEL_FAST, KERNEL_FAST_WIDE, KERNEL_COMBINED, KERNEL_RAW, KERNEL_QUAD = 1, 2, 4, 8, 16
 QUEUE_NONE, QUEUE_STREAM, QUEUE_CAPTURE, QUEUE_LEASE, QUEUE_SCRATCH = 0, 1, 2, 3, 4
 QUEUE_NAMES = {0: "none", 1: "stream", 2: "capture", 3: "lease", 4: "scratch"}
 
@@ -203,7 +203,7 @@ def last_launch() -> dict:
     check(_lib.navi_last_launch(ctypes.byref(info)))
     k = info.kernels
     return {"fast": bool(k & KERNEL_FAST), "fast_wide": bool(k & KERNEL_FAST_WIDE),
-            "combined": bool(k & KERNEL_COMBINED), "raw": bool(k & KERNEL_RAW),
+            "combined": bool(k & KERNEL_COMBINED), "raw": bool(k & KERNEL_RAW), "quad": bool(k & KERNEL_QUAD),
             "queue": QUEUE_NAMES.get(info.queue, str(info.queue)), "pair": info.pair,
             "fast_planes": info.fast_planes, "planes": info.planes, "staged": bool(info.staged),
             "waves": info.waves, "n_rays": info.n_rays}

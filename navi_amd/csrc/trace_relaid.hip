@@ -4,6 +4,8 @@
 // checkout); tests compare both against the CPU oracle bit for bit.
 //
 // Execution model (CDNA4, wave64):
+//   * launches below 2^19 rays: trace_quad_kernel, four lanes per ray
+//     (trace_quad.hpp); the rest below is about the larger ones;
 //   * two kernels: the fast march (monotone, tame, shallow scenes with split
 //     planes, the library compiler's) alone in trace_fast_kernel at eight
 //     waves per SIMD, in two 1024-thread workgroups per CU for launches of at
@@ -67,6 +69,9 @@ typedef uint32_t navi_u32x2 __attribute__((ext_vector_type(2)));
 extern "C" __device__ navi_u32x2 navi_struct_load_b64(__amdgpu_buffer_rsrc_t rsrc, int32_t index, int32_t voffset,
                                                        int32_t soffset, int32_t aux)
     __asm("llvm.amdgcn.struct.ptr.buffer.load.v2i32");
+
+// A lane mask with every set bit spread over its quad of lanes (s_wqm_b64).
+extern "C" __device__ uint64_t navi_s_wqm(uint64_t mask) __asm("llvm.amdgcn.s.wqm.i64");
 
 namespace navi {
 
@@ -143,6 +148,10 @@ struct RelaidParams {
     const uint32_t* __restrict__ leaves;
     uint32_t n_leaves;
     uint32_t sem_bits;
+    // trace_quad_kernel: units of 2^quad_shift rays, env_units of them per env
+    uint32_t quad_shift;
+    uint32_t env_units;
+    FastDiv div_units;  // by env_units
 };
 
 constexpr uint32_t kTableLeaf = 0xffff0000u;  // a leaf slot of the leaf table (low 16 bits: entry)
@@ -225,6 +234,9 @@ constexpr uint32_t kLeafRun = 1;  // leaf-cache steps taken after a leaf step
 // steps 1.5% faster than 1, refills at 12 idle lanes 1% faster than at 8).
 constexpr uint32_t kLeafRunFast = 2;
 constexpr uint32_t kRefillMinFast = 12;
+// The quad march's (trace_quad.hpp): 8, 4, 2 and 1 steps take 170, 159, 150 and
+// 155 us on 12 K rays of a 512^3 room grid (the wave waits for its longest run).
+constexpr uint32_t kQuadLeafRun = 2;
 // rays per dynamically claimed work unit (2 tiles): larger units leave more rays
 // held by one wave when the queue runs dry, smaller ones cost more claims
 constexpr uint32_t kUnitRays = 128;
@@ -277,19 +289,28 @@ constexpr size_t kFastLds = 20480;
 // their octants from the plane index: no midpoints, comparisons or selects).
 constexpr int kWideThreads = 1024;
 constexpr size_t kFastLdsWide = 81920;
-// Launches of fewer rays take the 256-thread workgroups: a small batch's few
-// workgroups then spread over more CUs (the wide grid holds as many waves, in
-// a quarter of the workgroups). Measured: 786 K rays on one 512^3 scene 3%
-// faster wide, 49 K rays 8% slower. navi_set_wide_min_rays changes it.
+// Launches of fewer rays take trace_quad_kernel or, with the threshold raised
+// (navi_set_wide_min_rays), from kFastMinRays on the 256-thread workgroups,
+// which spread a batch over more CUs (the wide grid holds as many waves, in a
+// quarter of the workgroups). Measured: 786 K rays on one 512^3 scene 3% faster
+// wide.
 constexpr uint64_t kWideMinRays = 1u << 19;
 std::atomic<uint64_t> g_wide_min_rays{kWideMinRays};
-// Launches of fewer rays skip the 256-thread fast kernel: the combined kernel
-// alone (its fast march at seven waves; such batches are bound by the latency
-// of their rays' chains, not by occupancy) saves the second launch (64^3 box
-// room 0.054 -> 0.053 ms, 49 K rays 0.111 -> 0.108 ms). With the default wide
-// threshold every larger launch whose planes fit takes the wide shape; the
-// 256-thread fast kernel serves launches between this and a raised one.
+// Launches of fewer rays skip the 256-thread fast kernel (a lowered wide
+// threshold whose planes do not fit): the combined kernel alone saves the
+// second launch.
 constexpr uint32_t kFastMinRays = 1u << 19;
+// Smaller launches (also than the wide threshold) take trace_quad_kernel, four
+// lanes per ray: they last as long as their longest rays' chains of steps, and
+// a quad's step takes about two thirds of the time (49 K rays on a 128^3 volume
+// 112 -> 72 us, 12 K on a 512^3 room grid 243 -> 150 us, 393 K there 433 -> 336
+// us). From about a million rays on the work counts: 1.57 M rays of 16 scenes
+// take 899 us in quads, 815 us a lane each.
+constexpr uint32_t kQuadMaxRays = 1u << 19;
+// ... and the smallest of those in units of 4 rays, which wait less on each
+// other and reach more CUs (12 K rays: 150 us, 159 in units of 16; 49 K rays:
+// no difference, at four times the waves).
+constexpr uint32_t kQuadSmallRays = 1u << 14;
 __host__ __device__ constexpr uint32_t axis_stride(uint32_t depth) { return (1u << depth) + 2u; }
 constexpr uint32_t kPlaneHeader = 8;  // floats before the planes: scales, pad, offsets, pad
 __host__ __device__ constexpr uint32_t scene_stride(uint32_t depth) {
@@ -1393,6 +1414,12 @@ __device__ __forceinline__ void march(const RelaidParams& P, SceneLds* lds_scene
     }
 }
 
+}  // namespace navi
+
+#include "trace_quad.hpp"
+
+namespace navi {
+
 // A workgroup's set-up: the scene table (and with kPD > 0 the split planes of
 // kPD levels) staged in LDS, and the launch-wide conditions, the same in every
 // workgroup.
@@ -1781,9 +1808,42 @@ int plane_depth_wide(int32_t n_scenes, uint32_t D, size_t budget) {
 // kernel traced it (every other launch: trace_relaid_kernel alone).
 int launch_relaid_queued(RelaidParams P, hipStream_t stream, uint32_t* scratch_queue, navi_launch_info& info);
 
+// A small batch on trace_quad_kernel: one wave per unit, no work queue (and no
+// queue pair: launches on any streams, captured or not, share nothing).
+int launch_quad(RelaidParams P, hipStream_t stream, navi_launch_info& info) {
+    const uint32_t D = P.cell_depth;
+    const bool poses = P.local_dirs != nullptr;
+    P.quad_shift = P.n_rays <= kQuadSmallRays ? 2u : 4u;
+    const uint32_t unit = 1u << P.quad_shift;
+    P.env_units = P.tile_el ? P.rays_per_env >> P.quad_shift : (P.rays_per_env + unit - 1u) / unit;
+    P.div_units = make_fastdiv(P.env_units);
+    const uint32_t blocks = P.n_envs * P.env_units;
+    void (*kernel)(RelaidParams) = nullptr;
+    switch (D) {
+        case 4: kernel = poses ? trace_quad_kernel<4, true> : trace_quad_kernel<4, false>; break;
+        case 5: kernel = poses ? trace_quad_kernel<5, true> : trace_quad_kernel<5, false>; break;
+        case 6: kernel = poses ? trace_quad_kernel<6, true> : trace_quad_kernel<6, false>; break;
+        default: kernel = poses ? trace_quad_kernel<7, true> : trace_quad_kernel<7, false>; break;
+    }
+    info.kernels = NAVI_KERNEL_COMBINED | NAVI_KERNEL_QUAD;
+    info.planes = kQuadPlanes;
+    info.waves = blocks;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64), 0, stream, P);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return set_error(NAVI_E_LAUNCH, "kernel launch failed: %s", hipGetErrorString(err));
+    return NAVI_OK;
+}
+
 int launch_relaid(RelaidParams P, hipStream_t stream, uint32_t* scratch_queue = nullptr) {
     navi_launch_info info = {};
     info.n_rays = P.n_rays;
+    P.small_tables = (static_cast<uint64_t>(P.n_scenes) << (3u * P.cell_depth + 3u)) < (1ull << 32) ? 1u : 0u;
+    if (P.n_rays < kQuadMaxRays && P.n_rays < g_wide_min_rays.load(std::memory_order_relaxed)) {
+        info.pair = -1;
+        const int code = launch_quad(P, stream, info);
+        g_last_launch = info;
+        return code;
+    }
     QueueChoice c;
     if (scratch_queue != nullptr) {
         c.words = scratch_queue;
@@ -1805,7 +1865,6 @@ int launch_relaid_queued(RelaidParams P, hipStream_t stream, uint32_t* queue, na
     P.n_chunks = (P.n_rays + 63u) / 64u;
     P.queue = queue;
     const uint32_t D = P.cell_depth;
-    P.small_tables = (static_cast<uint64_t>(P.n_scenes) << (3u * D + 3u)) < (1ull << 32) ? 1u : 0u;
     const bool poses = P.local_dirs != nullptr;
     const bool leaves = P.leaves != nullptr;
     // counters another launch may have used: cleared first (a kernel node,

@@ -1,0 +1,44 @@
+"""GPU parity of the small-batch tracer (trace_quad_kernel, four lanes per ray) against the
+CPU oracle at the edges of its units: rays per env around 4 and 16, batches on both sides
+of its 4-ray units (2^14 rays) and of the 512 units that an XCD round spans, tiled and
+linear order, with its fast and its general march."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from tests.test_gpu_multiscene import _compare, _oracle_multi, _rays, _run, corpus  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def resident(gpu, corpus):  # noqa: F811
+    from navi_amd.multiscene import ResidentScenes
+
+    return ResidentScenes([(c.words, c.bbox_min_list, c.bbox_max) for c in corpus])
+
+
+# (envs, az, el, elevation_bins): 1 ray; 3, 15, 17 and 65 rays per env; a batch of 4-ray
+# tiles; 16-ray units, one more than 512 of them and a tiled batch
+SHAPES = [(1, 1, 1, 0), (5, 3, 1, 0), (7, 5, 3, 0), (3, 17, 1, 0), (2, 13, 5, 0), (4, 16, 8, 8), (30, 32, 17, 0),
+          (513, 16, 2, 0), (21, 32, 32, 32)]
+
+
+@pytest.mark.parametrize("max_distance", [30.0, 1200.0])
+@pytest.mark.parametrize("envs,az,el,bins", SHAPES)
+def test_quad_units_match_the_oracle(resident, corpus, envs, az, el, bins, max_distance):  # noqa: F811
+    from navi_amd import _native
+
+    env_scene, o, d = _rays(corpus, envs, az, el, seed=envs + az)
+    if envs > 2:
+        env_scene[1] = 99  # an unknown scene: NaN, semantic 0, no steps
+    ref = _oracle_multi([c.words for c in corpus], [c.bbox_min_list + c.bbox_max for c in corpus],
+                        np.where(env_scene == 99, 0, env_scene).astype(np.int32), o, d, 160, max_distance)
+    if envs > 2:
+        ref["distance"][1], ref["semantic"][1], ref["steps"][1] = np.nan, 0, 0
+    got = _run(resident, env_scene, o, d, 160, max_distance, elevation_bins=bins)
+    info = _native.last_launch()
+    assert info["quad"] and info["n_rays"] == envs * az * el, info
+    _compare(got, ref, max_distance, f"{envs}x{az}x{el}/{bins}/{max_distance}")
