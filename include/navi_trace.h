@@ -237,6 +237,38 @@ int navi_build_cell_table(const uint32_t* records, uint64_t n_records, uint32_t 
                           uint64_t* out_table);
 
 /*
+ * The record layout made on the device (no reference counterpart): the arrays
+ * of navi_relayout and navi_build_cell_table, bit for bit, from DAG words in
+ * device memory. navi_relayout_device numbers the records and waits for its
+ * stream (an error while the stream is capturing): mark and order are device
+ * buffers of n_words u32 each, state one of NAVI_RELAYOUT_STATE_WORDS u32, all
+ * three scratch for the call and its navi_relayout_device_records.
+ * layout->converted is 0 for a DAG that is left to the host's conversion: a
+ * one-leaf DAG, a reachable leaf of semantic 0x7fff or above, more than 31
+ * levels of records, a record that is reached at two depths (a cycle among
+ * them), or 2^28 words and more. Else n_records, max_depth (navi_record_depth)
+ * and flags (navi_scene_flags) describe the scene, and
+ * navi_relayout_device_records writes its records, child records as pool
+ * indices from rec_offset on, without waiting.
+ */
+#define NAVI_RELAYOUT_STATE_WORDS 1088u
+typedef struct navi_device_layout {
+    uint32_t converted;
+    uint32_t n_records;
+    uint32_t max_depth;
+    uint32_t flags;
+} navi_device_layout;
+
+int navi_relayout_device(const uint64_t* words, uint64_t n_words, uint32_t* mark, uint32_t* order, uint32_t* state,
+                         navi_device_layout* layout, void* stream);
+int navi_relayout_device_records(const uint64_t* words, uint64_t n_words, const uint32_t* mark,
+                                 const uint32_t* order, uint32_t n_records, uint32_t rec_offset,
+                                 uint32_t* out_records, void* stream);
+/* navi_build_cell_table over records in device memory, into out_table there; does not wait. */
+int navi_build_cell_table_device(const uint32_t* records, uint64_t n_records, uint32_t root_slot, int32_t depth,
+                                 uint64_t* out_table, void* stream);
+
+/*
  * Throughput tracer over the device layout: n_envs * rays_per_env rays, env e
  * traces scenes[env_scene ? env_scene[e] : 0] (at most 1024 scenes; `records`
  * holds n_records records with absolute child slots, see navi_relaid_scene;

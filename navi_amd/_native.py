@@ -143,6 +143,22 @@ class LaunchInfo(ctypes.Structure):
                 ("waves", ctypes.c_uint32), ("n_rays", ctypes.c_uint64)]
 
 
+class DeviceLayout(ctypes.Structure):
+    """navi_device_layout (include/navi_trace.h)."""
+
+    _fields_ = [("converted", ctypes.c_uint32), ("n_records", ctypes.c_uint32), ("max_depth", ctypes.c_uint32),
+                ("flags", ctypes.c_uint32)]
+
+
+RELAYOUT_STATE_WORDS = 1088  # NAVI_RELAYOUT_STATE_WORDS (include/navi_trace.h)
+_lib.navi_relayout_device.restype = ctypes.c_int
+_lib.navi_relayout_device.argtypes = [_vp, ctypes.c_uint64, _vp, _vp, _vp, ctypes.POINTER(DeviceLayout), _vp]
+_lib.navi_relayout_device_records.restype = ctypes.c_int
+_lib.navi_relayout_device_records.argtypes = [_vp, ctypes.c_uint64, _vp, _vp, ctypes.c_uint32, ctypes.c_uint32, _vp,
+                                              _vp]
+_lib.navi_build_cell_table_device.restype = ctypes.c_int
+_lib.navi_build_cell_table_device.argtypes = [_vp, ctypes.c_uint64, ctypes.c_uint32, ctypes.c_int32, _vp, _vp]
+
 _lib.navi_trace_relaid_ex.restype = ctypes.c_int
 _lib.navi_trace_relaid_ex.argtypes = [ctypes.POINTER(RelaidLaunch), _vp]
 _lib.navi_last_launch.restype = ctypes.c_int

@@ -89,8 +89,8 @@ class ResidentScenes:
     """Concatenated word pool + scene table on one device.
 
     ``scenes`` is a sequence of ``(words, bbox_min, bbox_max)`` with ``words`` a
-    uint64 (or int64-viewed) array in the reference word layout; child pointers
-    stay relative to each scene's first word.
+    uint64 (or int64-viewed) array in the reference word layout, or an int64 tensor of
+    them on the device; child pointers stay relative to each scene's first word.
     """
 
     def __init__(self, scenes: Sequence[tuple[np.ndarray, Sequence[float], Sequence[float]]],
@@ -105,85 +105,41 @@ class ResidentScenes:
             self.device = torch.device("cuda", torch.cuda.current_device())
         table = np.zeros(len(scenes), dtype=_native.SCENE_DESC_DTYPE)
         offset = 0
-        chunks = []
+        chunks = []  # uint64 arrays, or int64 tensors that are already on the device
         for i, (words, lo, hi) in enumerate(scenes):
-            w = np.ascontiguousarray(np.asarray(words).view(np.uint64).reshape(-1))
-            if w.size == 0:
+            if isinstance(words, torch.Tensor) and words.device == self.device and words.is_cuda:
+                w = words.detach().view(torch.int64).reshape(-1)
+                size = int(w.numel())
+            else:
+                w = np.ascontiguousarray(np.asarray(words).view(np.uint64).reshape(-1))
+                size = int(w.size)
+            if size == 0:
                 raise ValueError(f"scene {i} has no words")
             for k in range(3):
                 if not (math.isfinite(float(lo[k])) and math.isfinite(float(hi[k])) and float(lo[k]) < float(hi[k])):
                     raise ValueError(f"scene {i}: bbox_min must be finite and strictly below bbox_max")
             table[i]["word_offset"] = offset
-            table[i]["n_words"] = w.size
+            table[i]["n_words"] = size
             table[i]["bbox_min"] = np.asarray(lo, np.float32)
             table[i]["bbox_max"] = np.asarray(hi, np.float32)
             chunks.append(w)
-            offset += w.size
+            offset += size
         self.n_scenes = len(scenes)
-        self.word_counts = [int(c.size) for c in chunks]
+        self.word_counts = [int(n) for n in table["n_words"]]
         self.host_table = table
         # the word pool serves kernel="raw"; callers that keep their own word tensor skip it
-        self.pool = torch.from_numpy(np.concatenate(chunks).view(np.int64)).to(self.device) if keep_words else None
+        self.pool = None
+        if keep_words:
+            self.pool = torch.empty(offset, dtype=torch.int64, device=self.device)
+            for w, at, n in zip(chunks, table["word_offset"], self.word_counts):
+                self.pool[int(at):int(at) + n] = self._words(w)
         self.table = torch.from_numpy(table.view(np.uint8).copy()).to(self.device)
 
-        # device record layout (one 32-byte record per internal node); leaves of
-        # semantic 0x7fff or above go to one leaf table shared by the pool
-        rtable = np.zeros(len(scenes), dtype=_native.RELAID_SCENE_DTYPE)
-        recs = []
-        leaf_tables = []
-        roff = 0
-        loff = 0
-        self.relaid_ok = True
-        for i, w in enumerate(chunks):
-            try:
-                rec, root, _levels, leaves = _native.relayout_leaves(w)
-                rec, root = _native.rebase_leaves(rec, root, loff)
-            except RuntimeError:
-                self.relaid_ok = False
-                break
-            leaf_tables.append(leaves)
-            loff += int(leaves.size)
-            rtable[i]["rec_offset"] = roff
-            rtable[i]["n_records"] = rec.shape[0]
-            # child record slots become absolute pool indices
-            rec = rec.copy()
-            child = rec < 0x7FFFFFFD
-            rec[child] += np.uint32(roff)
-            rtable[i]["root_slot"] = root if root & 0x80000000 else roff + root
-            rtable[i]["bbox_min"] = table[i]["bbox_min"]
-            rtable[i]["bbox_max"] = table[i]["bbox_max"]
-            recs.append(rec)
-            roff += rec.shape[0]
-        if self.relaid_ok:
-            # navi_trace_relaid reads the pool through a buffer resource whose
-            # 32-bit byte size must not wrap: fewer than 2^27 records
-            if roff >= (1 << 27):
-                self.relaid_ok = False
+        # device record layout (one 32-byte record per internal node), made on the
+        # device where its conversion covers every scene, else on the host
         self.n_leaves = 0
         self.leaves = None
-        if self.relaid_ok:
-            allrec = np.concatenate(recs) if roff else np.zeros((1, 8), np.uint32)
-            all_leaves = np.concatenate(leaf_tables) if loff else np.zeros(0, np.uint32)
-            for i in range(len(scenes)):
-                rtable[i]["max_depth"] = _native.record_depth(allrec[:roff], int(rtable[i]["root_slot"]))
-                rtable[i]["flags"] = _native.scene_flags(allrec[:roff], int(rtable[i]["root_slot"]), all_leaves)
-            if loff:
-                self.n_leaves = loff
-                self.leaves = torch.from_numpy(all_leaves.view(np.int32).copy()).to(self.device)
-            if table_depth is not None:
-                self.table_depth = int(table_depth)
-            else:
-                # no deeper than one level below the deepest record: such a table
-                # already answers every descent
-                deepest = max(int(d) for d in rtable["max_depth"])  # 0xffffffff for a cycle
-                self.table_depth = max(4, min(default_table_depth(len(scenes)), deepest + 1))
-            tables = np.concatenate([_native.cell_table(allrec[:roff], int(rtable[i]["root_slot"]), self.table_depth)
-                                     for i in range(len(scenes))])
-            self.cell_tables = torch.from_numpy(tables.view(np.int64)).to(self.device)
-            self.n_records = int(roff)
-            self.records = torch.from_numpy(allrec.view(np.int32).reshape(-1).copy()).to(self.device)
-            self.relaid_table = torch.from_numpy(rtable.view(np.uint8).copy()).to(self.device)
-            self.record_counts = [int(r.shape[0]) for r in recs]
+        self.relaid_ok = self._layout_on_device(chunks, table_depth) or self._layout_on_host(chunks, table_depth)
         self._order_key = None
         self._order = None
         # scene order by measured cost (module docstring)
@@ -208,6 +164,122 @@ class ResidentScenes:
             _native.device_init(self.device)
             with torch.cuda.device(self.device):
                 self._cost_event = torch.cuda.Event()
+
+    # ---- the record layout ----
+
+    @staticmethod
+    def _words(chunk: Any) -> torch.Tensor:
+        return chunk if isinstance(chunk, torch.Tensor) else torch.from_numpy(chunk.view(np.int64))
+
+    def _table_depth_for(self, rtable: np.ndarray, table_depth: int | None) -> int:
+        if table_depth is not None:
+            return int(table_depth)
+        # no deeper than one level below the deepest record: such a table
+        # already answers every descent
+        deepest = max(int(d) for d in rtable["max_depth"])  # 0xffffffff for a cycle
+        return max(4, min(default_table_depth(self.n_scenes), deepest + 1))
+
+    def _new_rtable(self) -> np.ndarray:
+        rtable = np.zeros(self.n_scenes, dtype=_native.RELAID_SCENE_DTYPE)
+        rtable["bbox_min"] = self.host_table["bbox_min"]
+        rtable["bbox_max"] = self.host_table["bbox_max"]
+        return rtable
+
+    def _layout_on_device(self, chunks: list, table_depth: int | None) -> bool:
+        """Records and cell tables converted on the device (``navi_relayout_device``), the
+        same arrays as the host's; False when it leaves a scene to the host. Waits for the
+        device: the arrays are complete for every stream when it returns."""
+        if self.device.type != "cuda":
+            return False
+        lib = _native.lib()
+        rtable = self._new_rtable()
+        pools = []
+        offset = 0
+        with torch.cuda.device(self.device):
+            current = torch.cuda.current_stream(self.device)
+            stream = current.cuda_stream
+            state = torch.empty(_native.RELAYOUT_STATE_WORDS, dtype=torch.int32, device=self.device)
+            for i, chunk in enumerate(chunks):
+                n, at = self.word_counts[i], int(self.host_table[i]["word_offset"])
+                words = self.pool[at:at + n] if self.pool is not None else self._words(chunk).to(self.device)
+                mark, order = (torch.empty(n, dtype=torch.int32, device=self.device) for _ in range(2))
+                layout = _native.DeviceLayout()
+                _native.check(lib.navi_relayout_device(words.data_ptr(), n, mark.data_ptr(), order.data_ptr(),
+                                                       state.data_ptr(), ctypes.byref(layout), stream))
+                # a pool holds fewer than 2^27 records (_layout_on_host)
+                if not layout.converted or offset + layout.n_records >= (1 << 27):
+                    return False
+                records = torch.empty(8 * layout.n_records, dtype=torch.int32, device=self.device)
+                _native.check(lib.navi_relayout_device_records(words.data_ptr(), n, mark.data_ptr(), order.data_ptr(),
+                                                               layout.n_records, offset, records.data_ptr(), stream))
+                pools.append(records)
+                rtable[i]["rec_offset"] = rtable[i]["root_slot"] = offset
+                rtable[i]["n_records"] = layout.n_records
+                rtable[i]["max_depth"] = layout.max_depth
+                rtable[i]["flags"] = layout.flags
+                offset += layout.n_records
+            self.table_depth = self._table_depth_for(rtable, table_depth)
+            self.records = torch.cat(pools) if len(pools) > 1 else pools[0]
+            self.n_records = offset
+            cells = 8 ** self.table_depth
+            self.cell_tables = torch.empty(self.n_scenes * cells, dtype=torch.int64, device=self.device)
+            for i in range(self.n_scenes):
+                _native.check(lib.navi_build_cell_table_device(
+                    self.records.data_ptr(), self.n_records, int(rtable[i]["root_slot"]), self.table_depth,
+                    self.cell_tables.data_ptr() + 8 * cells * i, stream))
+            self.relaid_table = torch.from_numpy(rtable.view(np.uint8).copy()).to(self.device)
+            self.record_counts = [int(c) for c in rtable["n_records"]]
+            current.synchronize()
+        return True
+
+    def _layout_on_host(self, chunks: list, table_depth: int | None) -> bool:
+        """Records and cell tables converted on the host and uploaded; leaves of semantic
+        0x7fff or above go to one leaf table shared by the pool. False when the record
+        layout cannot hold the scenes."""
+        rtable = self._new_rtable()
+        recs = []
+        leaf_tables = []
+        roff = 0
+        loff = 0
+        for i, chunk in enumerate(chunks):
+            w = chunk.cpu().numpy().view(np.uint64) if isinstance(chunk, torch.Tensor) else chunk
+            try:
+                rec, root, _levels, leaves = _native.relayout_leaves(w)
+                rec, root = _native.rebase_leaves(rec, root, loff)
+            except RuntimeError:
+                return False
+            leaf_tables.append(leaves)
+            loff += int(leaves.size)
+            rtable[i]["rec_offset"] = roff
+            rtable[i]["n_records"] = rec.shape[0]
+            # child record slots become absolute pool indices
+            rec = rec.copy()
+            child = rec < 0x7FFFFFFD
+            rec[child] += np.uint32(roff)
+            rtable[i]["root_slot"] = root if root & 0x80000000 else roff + root
+            recs.append(rec)
+            roff += rec.shape[0]
+        # navi_trace_relaid reads the pool through a buffer resource whose
+        # 32-bit byte size must not wrap: fewer than 2^27 records
+        if roff >= (1 << 27):
+            return False
+        allrec = np.concatenate(recs) if roff else np.zeros((1, 8), np.uint32)
+        all_leaves = np.concatenate(leaf_tables) if loff else np.zeros(0, np.uint32)
+        for i in range(self.n_scenes):
+            rtable[i]["max_depth"] = _native.record_depth(allrec[:roff], int(rtable[i]["root_slot"]))
+            rtable[i]["flags"] = _native.scene_flags(allrec[:roff], int(rtable[i]["root_slot"]), all_leaves)
+        if loff:
+            self.n_leaves = loff
+            self.leaves = torch.from_numpy(all_leaves.view(np.int32).copy()).to(self.device)
+        self.table_depth = self._table_depth_for(rtable, table_depth)
+        tables = np.concatenate([_native.cell_table(allrec[:roff], int(rtable[i]["root_slot"]), self.table_depth)
+                                 for i in range(self.n_scenes)])
+        self.cell_tables = torch.from_numpy(tables.view(np.int64)).to(self.device)
+        self.n_records = int(roff)
+        self.records = torch.from_numpy(allrec.view(np.int32).reshape(-1).copy()).to(self.device)
+        self.relaid_table = torch.from_numpy(rtable.view(np.uint8).copy()).to(self.device)
+        self.record_counts = [int(r.shape[0]) for r in recs]
+        return True
 
     @property
     def pool_bytes(self) -> int:

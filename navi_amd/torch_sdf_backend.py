@@ -20,12 +20,13 @@ even (record-layout tracer only; a call that would take the word-layout kernel r
 
 Kernels. ``kernel="auto"`` (default) traces with the record-layout tracer
 (``navi_trace_relaid``) over a record-layout copy of the DAG tensor: its words
-copied to the host once, converted (``navi_relayout``, ``navi_build_cell_table``)
-and uploaded, keyed by the tensor object, its version counter (in-place tensor
-ops invalidate it), its address and the bbox. ``prepare(dag_tensor, bbox_min,
+converted once, on the device (``navi_relayout_device``; the DAGs that it leaves
+to the host's ``navi_relayout_leaves`` are copied there and back), keyed by the
+tensor object, its version counter (in-place tensor ops invalidate it), its
+address and the bbox. ``prepare(dag_tensor, bbox_min,
 bbox_max)`` does that at scene load (the reference's ``_load_scene``,
 ``sdfdag_backend.py:1893-1900``); otherwise the first ``cast_rays`` with the
-tensor does it, with a device-to-host copy that waits for the device, and warns
+tensor does it, with allocations and waits for the device, and warns
 (``LayoutConversionWarning``, once per call site under Python's default warning
 filter; ``conversion_counts()`` counts every conversion). Writes
 that bypass the version counter (through ``.data``, or from outside PyTorch)
@@ -65,8 +66,8 @@ __all__ = ["cast_rays", "prepare", "invalidate", "conversion_counts", "LayoutCon
 
 
 class LayoutConversionWarning(RuntimeWarning):
-    """``cast_rays`` converted a DAG tensor to the record layout inside the call: a
-    device-to-host copy that waits for the device, a host relayout and an upload.
+    """``cast_rays`` converted a DAG tensor to the record layout inside the call: allocations
+    and waits for the device, and for some DAGs a host conversion and an upload.
     ``prepare()`` at scene load moves that work out of the step."""
 
 
@@ -165,8 +166,7 @@ class _RecordLayout:
         self.version = dag_tensor._version
         self.data_ptr = dag_tensor.data_ptr()
         self.bounds = bounds
-        words = dag_tensor.detach().cpu().numpy().view(np.uint64)
-        scenes = ResidentScenes([(words, bounds[0], bounds[1])], dag_tensor.device, keep_words=False)
+        scenes = ResidentScenes([(dag_tensor, bounds[0], bounds[1])], dag_tensor.device, keep_words=False)
         self.scenes = scenes if scenes.relaid_ok else None
 
     def valid_for(self, dag_tensor: torch.Tensor, bounds) -> bool:
@@ -192,7 +192,7 @@ def _record_layout(dag_tensor: torch.Tensor, bbox_min, bbox_max, caller: str):
             if caller == "cast_rays":
                 warnings.warn(
                     f"cast_rays converted a {dag_tensor.numel()}-word DAG tensor to the record layout inside the "
-                    "call (a device-to-host copy that waits for the device); call torch_sdf.prepare(dag_tensor, "
+                    "call (which allocates and waits for the device); call torch_sdf.prepare(dag_tensor, "
                     "bbox_min, bbox_max) when the scene is loaded", LayoutConversionWarning, stacklevel=4)
         return entry.scenes
 
