@@ -269,6 +269,15 @@ int navi_build_cell_table_device(const uint32_t* records, uint64_t n_records, ui
                                  uint64_t* out_table, void* stream);
 
 /*
+ * A quick form of the direction check (bindings.cpp:23-34): flags, n_flags
+ * device words, are all 0 when each of the n_dirs float3 directions is finite
+ * with a norm within 1e-4 of one by a margin (2e-6) that covers any order of
+ * rounding; a word of 1 leaves the decision to an exact check. n_flags is the
+ * launch's workgroups (about n_dirs / 256, any number works). Does not wait.
+ */
+int navi_check_directions(const float* dirs, int64_t n_dirs, uint32_t* flags, int32_t n_flags, void* stream);
+
+/*
  * Throughput tracer over the device layout: n_envs * rays_per_env rays, env e
  * traces scenes[env_scene ? env_scene[e] : 0] (at most 1024 scenes; `records`
  * holds n_records records with absolute child slots, see navi_relaid_scene;

@@ -159,6 +159,9 @@ _lib.navi_relayout_device_records.argtypes = [_vp, ctypes.c_uint64, _vp, _vp, ct
 _lib.navi_build_cell_table_device.restype = ctypes.c_int
 _lib.navi_build_cell_table_device.argtypes = [_vp, ctypes.c_uint64, ctypes.c_uint32, ctypes.c_int32, _vp, _vp]
 
+_lib.navi_check_directions.restype = ctypes.c_int
+_lib.navi_check_directions.argtypes = [_vp, ctypes.c_int64, _vp, ctypes.c_int32, _vp]
+
 _lib.navi_trace_relaid_ex.restype = ctypes.c_int
 _lib.navi_trace_relaid_ex.argtypes = [ctypes.POINTER(RelaidLaunch), _vp]
 _lib.navi_last_launch.restype = ctypes.c_int

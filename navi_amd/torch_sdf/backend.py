@@ -16,10 +16,12 @@ from typing import Any
 import torch
 
 torch_sdf_backend: Any | None = None
+_directions_within_tolerance: Any = lambda dirs: False  # noqa: E731
 try:
     from .. import torch_sdf_backend as _torch_sdf_backend
 
     torch_sdf_backend = _torch_sdf_backend
+    _directions_within_tolerance = _torch_sdf_backend.directions_within_tolerance
     HAS_CUDA_BACKEND = True
 except ImportError:
     HAS_CUDA_BACKEND = False
@@ -49,8 +51,11 @@ def _validate_cuda_tensor(tensor: Any, *, name: str, dtype: torch.dtype,
         raise RuntimeError(f"{name} must have shape {shape}; got {_shape_tuple(tensor)}.")
 
 
-def _validate_direction_norms(dirs: torch.Tensor, *, eps: float = _DIRECTION_NORM_EPS) -> None:
-    # backend.py:101-111
+def _validate_direction_norms(dirs: torch.Tensor, *, eps: float = _DIRECTION_NORM_EPS) -> bool:
+    # backend.py:101-111; returns whether one pass on the device was enough, by a margin
+    # that covers the native layer's own check (bindings.cpp:23-34) of the same tensor
+    if eps >= _DIRECTION_NORM_EPS and _directions_within_tolerance(dirs):
+        return True
     norms = torch.linalg.vector_norm(dirs, dim=-1)
     if bool((~torch.isfinite(norms)).any().item()):
         raise RuntimeError("dirs must contain only finite direction vectors.")
@@ -59,11 +64,12 @@ def _validate_direction_norms(dirs: torch.Tensor, *, eps: float = _DIRECTION_NOR
         raise RuntimeError(
             f"dirs must be normalized within tolerance {eps}; max error was {max_error:.6g}."
         )
+    return False
 
 
 def _validate_cast_rays_inputs(dag_tensor: Any, origins: Any, dirs: Any, out_distances: Any,
-                               out_semantics: Any, *, skip_direction_validation: bool = False) -> None:
-    # backend.py:49-98
+                               out_semantics: Any, *, skip_direction_validation: bool = False) -> bool:
+    # backend.py:49-98; returns whether the native layer may skip its direction check
     if not dag_tensor.is_cuda:
         raise RuntimeError("dag_tensor must be on CUDA. CPU tensors are not supported.")
     if dag_tensor.dtype != _DAG_DTYPE:
@@ -92,7 +98,8 @@ def _validate_cast_rays_inputs(dag_tensor: Any, origins: Any, dirs: Any, out_dis
     _validate_cuda_tensor(out_semantics, name="out_semantics", dtype=_SEMANTIC_DTYPE,
                           shape=(batch, rays))
     if not skip_direction_validation and torch.is_tensor(dirs):
-        _validate_direction_norms(dirs)
+        return _validate_direction_norms(dirs)
+    return skip_direction_validation
 
 
 def _validate_bounds(bbox_min: list[float], bbox_max: list[float]) -> None:
@@ -157,8 +164,9 @@ def cast_rays(
         raise RuntimeError(
             "CUDA is not available. TopoNav requires a ROCm GPU and does not support CPU fallback."
         )
-    _validate_cast_rays_inputs(dag_tensor, origins, dirs, out_distances, out_semantics,
-                               skip_direction_validation=skip_direction_validation)
+    skip_direction_validation = _validate_cast_rays_inputs(
+        dag_tensor, origins, dirs, out_distances, out_semantics,
+        skip_direction_validation=skip_direction_validation)
     _validate_runtime_parameters(max_steps=max_steps, max_distance=max_distance, bbox_min=bbox_min,
                                  bbox_max=bbox_max, resolution=resolution)
     backend = torch_sdf_backend

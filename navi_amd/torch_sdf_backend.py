@@ -93,7 +93,25 @@ def _validate_bounds(bbox_min, bbox_max) -> None:  # bindings.cpp:10-21
         _check(lo < hi, "bbox_min entries must be strictly less than bbox_max entries")
 
 
+def directions_within_tolerance(dirs: torch.Tensor) -> bool:
+    """Whether one pass on the device (``navi_check_directions``) finds every direction
+    finite and its norm within the tolerance, by a margin that any order of rounding fits
+    in. False leaves the decision to the exact checks (also for tensors the kernel does not
+    take: CPU, other types or layouts, none at all). Waits for the device."""
+    if not (type(dirs) is torch.Tensor and dirs.is_cuda and dirs.dtype == torch.float32 and dirs.is_contiguous()
+            and dirs.dim() >= 1 and dirs.size(-1) == 3 and dirs.numel() > 0):
+        return False
+    n = dirs.numel() // 3
+    flags = torch.empty(min(256, -(-n // 256)), dtype=torch.int32, device=dirs.device)
+    with torch.cuda.device(dirs.device):
+        stream = torch.cuda.current_stream(dirs.device).cuda_stream
+        _native.check(_native.lib().navi_check_directions(dirs.data_ptr(), n, flags.data_ptr(), flags.numel(), stream))
+        return not flags.cpu().numpy().any()
+
+
 def _validate_direction_norms(dirs: torch.Tensor) -> None:  # bindings.cpp:23-34
+    if directions_within_tolerance(dirs):
+        return
     norms = torch.sqrt(torch.sum(dirs * dirs, -1))
     _check(bool(torch.isfinite(norms).all().item()), "dirs must contain only finite direction vectors")
     max_error = float(torch.abs(norms - 1.0).amax().item())
