@@ -57,6 +57,8 @@ __device__ __forceinline__ uint32_t quad_min(uint32_t x) {
 
 // The quads (every lane of them) with a set bit in m.
 __device__ __forceinline__ uint64_t quad_any(uint64_t m) { return navi_s_wqm(m); }
+// The quads with no set bit in m.
+__device__ __forceinline__ uint64_t quad_none(uint64_t m) { return ~quad_any(m); }
 // The quads whose axis lanes all have their bit set in m.
 __device__ __forceinline__ uint64_t quad_all(uint64_t m) { return ~quad_any(~m & kAxisLanes); }
 
@@ -133,7 +135,10 @@ __device__ __forceinline__ QuadResult quad_fast(const RelaidParams& P, const nav
     const float nan = __builtin_nanf("");
     const uint64_t neg = wave_mask(__float_as_int(d) < 0 && axis != 3u);  // the mirrored axes
     const bool inside = lane_in(quad_all(wave_mask(o >= lo_a && o <= hi_a)));
-    float dm = inside ? (lane_in(neg) ? -lo_a : hi_a) : nan;  // the domain's face ahead
+    // the domain's face ahead; lane 3's faces are at +inf and its q' is 0, so it
+    // passes every test of the march and the tests need not leave it out
+    constexpr float kInf = __builtin_inff();
+    const float dm = axis == 3u ? kInf : (inside ? (lane_in(neg) ? -lo_a : hi_a) : nan);
     const float ad = fabsf(d);
     const float r = (axis != 3u && (d > kDirEps || d < -kDirEps)) ? fabsf(1.0f / d) : nan;
     // lane 3's sample is -FLT_MAX (q' = 0 with the flip's bits): it lies below
@@ -141,6 +146,7 @@ __device__ __forceinline__ QuadResult quad_fast(const RelaidParams& P, const nav
     scale = axis == 3u ? 0.f : scale;
     off = axis == 3u ? 0.f : off;
     const uint32_t flip = axis == 3u ? 0xff7fffffu : (lane_in(neg) ? 0x80000000u : 0u);
+    const uint32_t face_keep = axis == 3u ? 0u : 0xffffffffu, face_flip = axis == 3u ? 0x7f800000u : flip;
     const float om = axis == 3u ? 0.f : mirror(o, d);
     const float adm = axis == 3u ? 0.f : ad;
     const float* const pl = planes + ax * kQuadAxis;
@@ -152,7 +158,7 @@ __device__ __forceinline__ QuadResult quad_fast(const RelaidParams& P, const nav
         static_cast<int>(static_cast<uint32_t>(P.n_scenes) << (3u * D)), 0x00020000);
     const uint32_t my_table = scene << (3u * D);
     const bool root_leaf = (S.root_slot & 0x80000000u) != 0u;  // a one-leaf DAG: its leaf is the domain
-    float lf = root_leaf ? dm : nan;                            // the cached leaf's face ahead
+    float lf = root_leaf || axis == 3u ? dm : nan;              // the cached leaf's face ahead
     uint32_t lf_slot = (P.leaves != nullptr && root_leaf) ? table_leaf_word(S.root_slot, P.leaves, P.n_leaves)
                                                           : S.root_slot;
     uint32_t pre = 0xffffffffu;  // the prefix cell's upper face along the axis, as a plane index
@@ -163,11 +169,11 @@ __device__ __forceinline__ QuadResult quad_fast(const RelaidParams& P, const nav
     while (live != 0ull) {
         step = add_lane_bit(step, live);
         const float qa = __builtin_fmaf(t, adm, om);
-        const uint64_t m_dom = quad_all(wave_mask(qa <= dm));
-        const uint64_t m_hit_lf = quad_all(wave_mask(qa <= lf)) & live;
+        const uint64_t m_dom = quad_none(wave_mask(!(qa <= dm)));
+        const uint64_t m_hit_lf = quad_none(wave_mask(!(qa <= lf))) & live;
         const uint64_t m_desc = live & m_dom & ~m_hit_lf;
         // (lanes that do not descend: void marker and a face at +inf, see march_fast)
-        float h = __builtin_inff();
+        float h = kInf;
         uint32_t slot = kSlotVoid;
         if (lane_in(m_desc)) {
             const float p = __uint_as_float(__float_as_uint(qa) ^ flip);
@@ -192,7 +198,7 @@ __device__ __forceinline__ QuadResult quad_fast(const RelaidParams& P, const nav
 #pragma unroll
             for (uint32_t l = 0; l < kUp; ++l)
                 w |= ((j >> (kUp - 1u - l)) & 1u) << (3u * (D + l) + ax);
-            w = quad_or(axis == 3u ? 0u : w);
+            w = quad_or(w);  // (lane 3's j is 0)
             const navi_u32x2 e = navi_struct_load_b64(
                 tables, static_cast<int32_t>(my_table | (w & ((1u << (3u * D)) - 1u))), 0, 0, 0);
             slot = e[0];
@@ -226,7 +232,7 @@ __device__ __forceinline__ QuadResult quad_fast(const RelaidParams& P, const nav
                 }
                 h = lane_in(neg) ? lo : hi;
             }
-            h = __uint_as_float(__float_as_uint(h) ^ flip);  // mirrored
+            h = __uint_as_float((__float_as_uint(h) & face_keep) ^ face_flip);  // mirrored
         }
 
         // ---- the query's outcome and the leaf cache ----
@@ -255,7 +261,7 @@ __device__ __forceinline__ QuadResult quad_fast(const RelaidParams& P, const nav
         // ---- further steps that the leaf cache answers alone ----
         uint64_t m_run = live & ~m_fin & m_leaf;
         for (uint32_t k = 0; k < kQuadLeafRun; ++k) {
-            m_run &= quad_all(wave_mask(__builtin_fmaf(t, adm, om) <= lf));
+            m_run &= quad_none(wave_mask(!(__builtin_fmaf(t, adm, om) <= lf)));
             if (m_run == 0ull) break;
             step = add_lane_bit(step, m_run);
             t = lane_in(m_run) ? t + dist : t;
