@@ -116,56 +116,51 @@ struct QuadResult {
     int32_t step, sem;
 };
 
-// The fast march of a wave's rays (march_fast, an axis a lane): box [lo_a, hi_a]
-// of scene S along the lane's axis with the plane lookup's scale and offset, the
-// ray's origin o and direction d along it.
-template <int kDepth>
-__device__ __forceinline__ QuadResult quad_fast(const RelaidParams& P, const navi_relaid_scene& S, uint32_t scene,
-                                                float lo_a, float hi_a, float scale, float off, float o, float d,
-                                                bool has_ray, float* planes) {
+// A ray's state as quad_march takes it, an axis a lane: the axis's plane lookup
+// (planes, scale, offset), mirrored origin and |direction|, exit reciprocal
+// (NaN on axes the exit leaves out), the faces ahead of the domain and of the
+// cached leaf (NaN: outside, none cached), the prefix cell's upper face as a
+// depth-8 plane index, and, the same in all four lanes, the cell table's first
+// entry, the leaf's word, t and the step count. Lane 3's om, adm, scale and off
+// are 0 and its dm and lf +inf.
+struct QuadRay {
+    const float* pl;
+    float scale, off, om, adm, r, dm, lf;
+    uint32_t pre, table, lf_slot;
+    float t;
+    int32_t step, sem;
+};
+
+// The fast march (march_fast, an axis a lane) of the rays of the quads in live
+// (whole quads, as every mask below) to their ends; neg holds the mirrored
+// axes. kLeaves: see march_fast.
+template <int kDepth, bool kLeaves>
+__device__ __forceinline__ void quad_march(const RelaidParams& P, uint64_t neg, uint64_t live, QuadRay& R) {
     constexpr uint32_t D = kDepth;
     constexpr uint32_t kUp = kQuadPlanes - D;  // levels between the table and the planes
     constexpr uint32_t kSh = kQuadPlanes - kPrefixDepth;
     constexpr uint32_t kCells = 1u << kQuadPlanes;
-    const uint32_t lane = threadIdx.x;
-    const uint32_t axis = lane & 3u;
-    const uint32_t ax = axis == 3u ? 0u : axis;
-    stage_quad_planes(S.bbox_min, S.bbox_max, lane, planes);
-    __syncthreads();
-    const float nan = __builtin_nanf("");
-    const uint64_t neg = wave_mask(__float_as_int(d) < 0 && axis != 3u);  // the mirrored axes
-    const bool inside = lane_in(quad_all(wave_mask(o >= lo_a && o <= hi_a)));
-    // the domain's face ahead; lane 3's faces are at +inf and its q' is 0, so it
-    // passes every test of the march and the tests need not leave it out
     constexpr float kInf = __builtin_inff();
-    const float dm = axis == 3u ? kInf : (inside ? (lane_in(neg) ? -lo_a : hi_a) : nan);
-    const float ad = fabsf(d);
-    const float r = (axis != 3u && (d > kDirEps || d < -kDirEps)) ? fabsf(1.0f / d) : nan;
+    const float nan = __builtin_nanf("");
+    const uint32_t axis = threadIdx.x & 3u;
+    const uint32_t ax = axis == 3u ? 0u : axis;
     // lane 3's sample is -FLT_MAX (q' = 0 with the flip's bits): it lies below
     // every plane and midpoint, so it adds no index or octant bit
-    scale = axis == 3u ? 0.f : scale;
-    off = axis == 3u ? 0.f : off;
     const uint32_t flip = axis == 3u ? 0xff7fffffu : (lane_in(neg) ? 0x80000000u : 0u);
     const uint32_t face_keep = axis == 3u ? 0u : 0xffffffffu, face_flip = axis == 3u ? 0x7f800000u : flip;
-    const float om = axis == 3u ? 0.f : mirror(o, d);
-    const float adm = axis == 3u ? 0.f : ad;
-    const float* const pl = planes + ax * kQuadAxis;
     const uint32_t ahead_up = lane_in(neg) ? 0u : 1u;
     const __amdgpu_buffer_rsrc_t records = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint32_t*>(P.records), static_cast<short>(4), static_cast<int>(P.n_records * 8u), 0x00020000);
     const __amdgpu_buffer_rsrc_t tables = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint64_t*>(P.cell_table), static_cast<short>(8),
         static_cast<int>(static_cast<uint32_t>(P.n_scenes) << (3u * D)), 0x00020000);
-    const uint32_t my_table = scene << (3u * D);
-    const bool root_leaf = (S.root_slot & 0x80000000u) != 0u;  // a one-leaf DAG: its leaf is the domain
-    float lf = root_leaf || axis == 3u ? dm : nan;              // the cached leaf's face ahead
-    uint32_t lf_slot = (P.leaves != nullptr && root_leaf) ? table_leaf_word(S.root_slot, P.leaves, P.n_leaves)
-                                                          : S.root_slot;
-    uint32_t pre = 0xffffffffu;  // the prefix cell's upper face along the axis, as a plane index
-    float t = 0.f;
-    int32_t step = 0, sem = 0;
+    const float* const pl = R.pl;
+    const float scale = R.scale, off = R.off, om = R.om, adm = R.adm, r = R.r, dm = R.dm;
+    const uint32_t my_table = R.table;
+    float lf = R.lf, t = R.t;
+    uint32_t pre = R.pre, lf_slot = R.lf_slot;
+    int32_t step = R.step, sem = 0;
 
-    uint64_t live = wave_mask(has_ray);  // whole quads, as every mask below
     while (live != 0ull) {
         step = add_lane_bit(step, live);
         const float qa = __builtin_fmaf(t, adm, om);
@@ -240,7 +235,7 @@ __device__ __forceinline__ QuadResult quad_fast(const RelaidParams& P, const nav
         const uint64_t m_leaf = m_hit_lf | m_new;
         lf = lane_in(m_new) ? h : lf;
         lf_slot = lane_in(m_new) ? slot : lf_slot;
-        if (P.leaves != nullptr && lane_in(m_new)) lf_slot = table_leaf_word(slot, P.leaves, P.n_leaves);
+        if (kLeaves && P.leaves != nullptr && lane_in(m_new)) lf_slot = table_leaf_word(slot, P.leaves, P.n_leaves);
 
         // ---- finish the step (kernel.cu:54-85, 297-308): an axis's quotient
         // clamped to [1e-5, 1000] (NaN to 1000) is a positive float, ordered as
@@ -271,7 +266,45 @@ __device__ __forceinline__ QuadResult quad_fast(const RelaidParams& P, const nav
         }
         live &= ~m_fin;
     }
-    return {t, step, sem};
+    R.t = t;
+    R.step = step;
+    R.sem = sem;
+}
+
+// The fast march of a wave's rays (march_fast, an axis a lane): box [lo_a, hi_a]
+// of scene S along the lane's axis with the plane lookup's scale and offset, the
+// ray's origin o and direction d along it.
+template <int kDepth>
+__device__ __forceinline__ QuadResult quad_fast(const RelaidParams& P, const navi_relaid_scene& S, uint32_t scene,
+                                                float lo_a, float hi_a, float scale, float off, float o, float d,
+                                                bool has_ray, float* planes) {
+    constexpr uint32_t D = kDepth;
+    const uint32_t lane = threadIdx.x;
+    const uint32_t axis = lane & 3u;
+    const uint32_t ax = axis == 3u ? 0u : axis;
+    stage_quad_planes(S.bbox_min, S.bbox_max, lane, planes);
+    __syncthreads();
+    const float nan = __builtin_nanf("");
+    constexpr float kInf = __builtin_inff();
+    const uint64_t neg = wave_mask(__float_as_int(d) < 0 && axis != 3u);  // the mirrored axes
+    const bool inside = lane_in(quad_all(wave_mask(o >= lo_a && o <= hi_a)));
+    const bool root_leaf = (S.root_slot & 0x80000000u) != 0u;  // a one-leaf DAG: its leaf is the domain
+    QuadRay R;
+    R.pl = planes + ax * kQuadAxis;
+    R.scale = axis == 3u ? 0.f : scale;
+    R.off = axis == 3u ? 0.f : off;
+    R.om = axis == 3u ? 0.f : mirror(o, d);
+    R.adm = axis == 3u ? 0.f : fabsf(d);
+    R.r = (axis != 3u && (d > kDirEps || d < -kDirEps)) ? fabsf(1.0f / d) : nan;
+    R.dm = axis == 3u ? kInf : (inside ? (lane_in(neg) ? -lo_a : hi_a) : nan);
+    R.lf = root_leaf || axis == 3u ? R.dm : nan;
+    R.lf_slot = (P.leaves != nullptr && root_leaf) ? table_leaf_word(S.root_slot, P.leaves, P.n_leaves) : S.root_slot;
+    R.pre = 0xffffffffu;
+    R.table = scene << (3u * D);
+    R.t = 0.f;
+    R.step = 0;
+    quad_march<kDepth, true>(P, neg, wave_mask(has_ray), R);
+    return {R.t, R.step, R.sem};
 }
 
 // The general march of a wave's rays (march in trace_relaid.hip, an axis a

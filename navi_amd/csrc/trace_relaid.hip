@@ -18,7 +18,8 @@
 //     tile for batches too small to fill the chip) from a counter pair of
 //     the launch's stream (or of the graph node it was captured into), the
 //     last wave rearming it; without a counter (all 4096 pairs in use) wave
-//     w takes 64-ray chunks w, w + W, ...;
+//     w takes 64-ray chunks w, w + W, ...; a wave of the fast kernel at plane
+//     depth 8 marches its last 16 rays with four lanes each (trace_quad.hpp);
 //   * lane refill: once 8 (fast march: 12) of 64 lanes have finished their rays, the idle lanes
 //     take the next rays (ballot + mbcnt rank), so a wave never idles on a few
 //     long rays;
@@ -532,6 +533,12 @@ __device__ __forceinline__ const RelaidParams& reload_params() {
     return *(const RelaidParams*)__builtin_amdgcn_kernarg_segment_ptr();  // address-space cast
 }
 
+}  // namespace navi
+
+#include "trace_quad.hpp"
+
+namespace navi {
+
 // The fast march: launches whose scenes all have split planes in LDS, tame
 // boxes, no record deeper than 30 levels and no negative leaf distance, with
 // cell tables below 4 GiB (every scene the library's compiler writes) and a
@@ -608,6 +615,8 @@ __device__ __forceinline__ void march_fast(const RelaidParams& P, const SceneLds
     // above the scene table, never at address 0) ----
     const bool stage = P.stage != 0u;
     const bool out_steps = P.out_steps != nullptr;
+    // a wave's last rays finish in quads (below) where the planes are the quads'
+    constexpr bool kQuadEnd = kPD == kQuadPlanes && !kLeaves;
     uint32_t tag = 0, ring = 0;
     uint32_t st0 = kNoTile, st1 = kNoTile;
     uint32_t* const my_stage = lds_stage + (threadIdx.x >> 6) * (kStageSlots * kStageWords);
@@ -644,6 +653,7 @@ __device__ __forceinline__ void march_fast(const RelaidParams& P, const SceneLds
     while (true) {
         // ---- refill idle lanes (as the general march) ----
         const uint32_t n_need = lane_count(need);
+        if (kQuadEnd && sched.exhausted && n_need >= 48u) break;
         if ((n_need >= kRefillMinFast || n_need == 64u) && !sched.exhausted) {
             const uint32_t rank = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(need >> 32),
                                                             __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(need), 0u));
@@ -958,6 +968,71 @@ __device__ __forceinline__ void march_fast(const RelaidParams& P, const SceneLds
             if (out_steps) {
                 const RelaidParams& RP = reload_params();
                 RP.out_steps[ray] = step;
+            }
+        }
+    }
+    // ---- the wave's last rays, at most 16, four lanes each: when the queue has
+    // run dry a launch lasts as long as the chains of steps of the rays still
+    // marching, and every wave issues a whole step for the few it has left;
+    // a quad's step issues a third of the vector instructions (786 K rays of a
+    // 512^3 room grid 577 -> 553 us, 1.57 M of 16 scenes 802 -> 774, 12.6 M of
+    // them 2674 -> 2653; registers and the loop before are unchanged) ----
+    if constexpr (kQuadEnd) {
+        const uint64_t last = ~need;
+        if (last != 0ull) {
+            const RelaidParams& RP = reload_params();
+            const uint32_t n = lane_count(last);
+            const uint32_t axis = lane & 3u;
+            // the lane that holds the quad's ray: the live lanes send their numbers
+            // to the quads' first lanes in turn (the others theirs to lane 63, which
+            // is no quad's first), and the quads spread them
+            const uint32_t rank = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(last >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(last), 0u));
+            const int32_t sent = __builtin_amdgcn_ds_permute(static_cast<int32_t>(lane_in(last) ? 16u * rank : 252u),
+                                                             static_cast<int32_t>(lane));
+            const int32_t from = 4 * __builtin_amdgcn_mov_dpp(sent, 0x00, 0xf, 0xf, true);
+            auto get = [&](uint32_t v) {
+                return static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(from, static_cast<int32_t>(v)));
+            };
+            auto get_axis = [&](float x, float y, float z) {
+                const uint32_t gx = get(__float_as_uint(x)), gy = get(__float_as_uint(y)), gz = get(__float_as_uint(z));
+                return __uint_as_float(axis == 1u ? gy : (axis == 2u ? gz : gx));
+            };
+            const float nan = __builtin_nanf("");
+            const uint32_t q_ray = get(ray), q_tag = get(tag), q_scene = get(scene);
+            const float* hdr = lds_planes + __umul24(q_scene, kScene);
+            const uint32_t ax = axis == 3u ? 0u : axis;
+            const float d = get_axis(dx, dy, dz);
+            const uint64_t neg = wave_mask(__float_as_int(d) < 0 && axis != 3u);
+            const float om = get_axis(ox, oy, oz), r = get_axis(rx, ry, rz);
+            const float dm = get_axis(dmx, dmy, dmz), lf = get_axis(lfx, lfy, lfz);
+            const uint32_t cell = get(pre_cell);
+            QuadRay R;
+            R.pl = hdr + kPlaneHeader + ax * kAxis;
+            R.scale = axis == 3u ? 0.f : hdr[ax];
+            R.off = axis == 3u ? 0.f : hdr[4u + ax];
+            R.om = axis == 3u ? 0.f : om;
+            R.adm = axis == 3u ? 0.f : fabsf(d);
+            R.r = axis == 3u ? nan : fabsf(r);
+            R.dm = axis == 3u ? __builtin_inff() : dm;
+            R.lf = axis == 3u ? __builtin_inff() : lf;
+            // (a field of ones, nothing cached, is no plane index)
+            R.pre = axis == 3u ? 0xffffffffu : (cell >> (kFW * axis)) & kFMask;
+            R.table = get(my_table);
+            R.lf_slot = get(lf_slot);
+            R.t = __uint_as_float(get(__float_as_uint(t)));
+            R.step = static_cast<int32_t>(get(static_cast<uint32_t>(step)));
+            quad_march<kDepth, kLeaves>(RP, neg, n >= 16u ? ~0ull : (1ull << (4u * n)) - 1ull, R);
+            if (axis == 0u && lane < 4u * n) {
+                if (q_tag != 0u) {
+                    lds_u32* e = lds_pointer(q_tag);
+                    e[0] = __float_as_uint(R.t);
+                    e[64] = static_cast<uint32_t>(R.sem);
+                } else {
+                    store_distance(RP, q_ray, R.t);
+                    __builtin_nontemporal_store(R.sem, &RP.out_s[q_ray]);
+                }
+                if (out_steps) RP.out_steps[q_ray] = R.step;
             }
         }
     }
@@ -1414,11 +1489,6 @@ __device__ __forceinline__ void march(const RelaidParams& P, SceneLds* lds_scene
     }
 }
 
-}  // namespace navi
-
-#include "trace_quad.hpp"
-
-namespace navi {
 
 // A workgroup's set-up: the scene table (and with kPD > 0 the split planes of
 // kPD levels) staged in LDS, and the launch-wide conditions, the same in every

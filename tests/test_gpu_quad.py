@@ -42,3 +42,27 @@ def test_quad_units_match_the_oracle(resident, corpus, envs, az, el, bins, max_d
     info = _native.last_launch()
     assert info["quad"] and info["n_rays"] == envs * az * el, info
     _compare(got, ref, max_distance, f"{envs}x{az}x{el}/{bins}/{max_distance}")
+
+
+# one wave with fewer than, exactly and more than 16 rays; envs of different scenes in one wave; several
+# waves; a tiled batch
+@pytest.mark.parametrize("envs,az,el,bins", SHAPES + [(1, 15, 1, 0), (1, 16, 1, 0), (16, 1, 1, 0), (33, 1, 2, 0)])
+@pytest.mark.parametrize("steps", [160, 7])
+def test_last_rays_of_a_wave_match_the_oracle(resident, corpus, envs, az, el, bins, steps):  # noqa: F811
+    """The one-lane-per-ray kernel, whose waves hand their last 16 rays to quads: rays
+    handed over before their first step, between steps, and close to the step limit."""
+    from navi_amd import _native
+
+    env_scene, o, d = _rays(corpus, envs, az, el, seed=envs + az)
+    o = o.copy()
+    o[0, 0] = [1e3, 1e3, 1e3]  # a ray from outside the domain
+    ref = _oracle_multi([c.words for c in corpus], [c.bbox_min_list + c.bbox_max for c in corpus],
+                        env_scene.astype(np.int32), o, d, steps, 30.0)
+    prev = _native.set_wide_min_rays(0)
+    try:
+        got = _run(resident, env_scene, o, d, steps, 30.0, elevation_bins=bins)
+        info = _native.last_launch()
+    finally:
+        _native.set_wide_min_rays(prev)
+    assert info["fast_wide"] and not info["quad"] and info["fast_planes"] == 8, info
+    _compare(got, ref, 30.0, f"{envs}x{az}x{el}/{bins}/{steps}")
