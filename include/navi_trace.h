@@ -394,10 +394,10 @@ int navi_trace_relaid_ex(const navi_relaid_launch* launch, void* stream);
  * Launch shape of the record-layout tracer (no reference counterpart: a tuning
  * knob of this library). Launches of at least `n_rays` rays whose scenes'
  * split planes fit two levels below the cell tables in 80 KiB of LDS run in
- * 1024-thread workgroups (two per CU), a lane per ray; smaller launches below
- * 2^19 rays run with four lanes per ray (trace_quad_kernel), smaller launches
- * of 2^19 rays and more in 256-thread workgroups. Results are identical either
- * way. Process-wide, thread-safe; takes effect from the next launch. Returns
+ * 1024-thread workgroups, a lane per ray; smaller launches below 2^19 rays run
+ * with four lanes per ray (trace_quad_kernel), smaller launches of 2^19 rays and
+ * more in 256-thread workgroups. At the default threshold launches below 851,968
+ * rays run with four lanes per ray. Results are identical either way. Process-wide, thread-safe; takes effect from the next launch. Returns
  * the previous value (default 2^19).
  */
 uint64_t navi_set_wide_min_rays(uint64_t n_rays);

@@ -4,7 +4,7 @@
 // checkout); tests compare both against the CPU oracle bit for bit.
 //
 // Execution model (CDNA4, wave64):
-//   * launches below 2^19 rays: trace_quad_kernel, four lanes per ray
+//   * launches below kQuadMaxRays rays: trace_quad_kernel, four lanes per ray
 //     (trace_quad.hpp); the rest below is about the larger ones;
 //   * two kernels: the fast march (monotone, tame, shallow scenes with split
 //     planes, the library compiler's) alone in trace_fast_kernel at eight
@@ -49,6 +49,7 @@
 // multiply-high division by the (uniform) rays-per-env and tile counts.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <map>
@@ -290,24 +291,34 @@ constexpr size_t kFastLds = 20480;
 // their octants from the plane index: no midpoints, comparisons or selects).
 constexpr int kWideThreads = 1024;
 constexpr size_t kFastLdsWide = 81920;
-// Launches of fewer rays take trace_quad_kernel or, with the threshold raised
-// (navi_set_wide_min_rays), from kFastMinRays on the 256-thread workgroups,
-// which spread a batch over more CUs (the wide grid holds as many waves, in a
-// quarter of the workgroups). Measured: 786 K rays on one 512^3 scene 3% faster
-// wide.
+// Launches of at least so many rays run wide where trace_quad_kernel does not take
+// them (kQuadMaxRays); with the threshold raised (navi_set_wide_min_rays), launches
+// below it take the 256-thread workgroups from kFastMinRays rays on, which spread
+// a batch over more CUs (786 K rays on one 512^3 scene 3% faster wide).
 constexpr uint64_t kWideMinRays = 1u << 19;
 std::atomic<uint64_t> g_wide_min_rays{kWideMinRays};
 // Launches of fewer rays skip the 256-thread fast kernel (a lowered wide
 // threshold whose planes do not fit): the combined kernel alone saves the
 // second launch.
 constexpr uint32_t kFastMinRays = 1u << 19;
-// Smaller launches (also than the wide threshold) take trace_quad_kernel, four
-// lanes per ray: they last as long as their longest rays' chains of steps, and
-// a quad's step takes about two thirds of the time (49 K rays on a 128^3 volume
-// 112 -> 72 us, 12 K on a 512^3 room grid 243 -> 150 us, 393 K there 433 -> 336
-// us). From about a million rays on the work counts: 1.57 M rays of 16 scenes
-// take 899 us in quads, 815 us a lane each.
-constexpr uint32_t kQuadMaxRays = 1u << 19;
+// Smaller launches take trace_quad_kernel, four lanes per ray (with the wide
+// threshold moved, those below it and below kFastMinRays): they last as long as
+// their longest rays' chains of steps, and a quad's step takes about two thirds of
+// the time (49 K rays on a 128^3 volume 112 -> 72 us, 12 K on a 512^3 room grid 243 ->
+// 150 us). From about a million rays on the work counts. Us in quads and a lane each
+// (the better of its two grids below): 836 K rays of 16 1024^3 scenes 524 and 570, of
+// a 512^3 room grid 538 and 517, of a 256^3 volume 355 and 325, of a 128^3 room 231
+// and 318; 688 K: 481 and 548, 459 and 475, 303 and 294, 205 and 295; 1.03 M: 637 and
+// 602, 610 and 572, 413 and 362, 283 and 346.
+constexpr uint32_t kQuadMaxRays = 13u << 16;
+// Wide launches of fewer rays run one workgroup per CU instead of two: a SIMD that
+// issues for four waves takes half the time per step, which shortens the chains that
+// such a launch ends on, and its waves refill twice as often. Us with one and two
+// workgroups: 1.03 M rays of 16 1024^3 scenes 602 and 617, of a 512^3 room grid 572 and
+// 593, of a 256^3 volume 362 and 437, of a 128^3 room 346 and 436; 1.57 M: 715 and 752,
+// 719 and 687, 472 and 541, 452 and 541; 3.1 M: 1164 and 1031, 1155 and 993, 738 and 813,
+// 729 and 821.
+constexpr uint32_t kOnePerCuRays = 5u << 18;
 // ... and the smallest of those in units of 4 rays, which wait less on each
 // other and reach more CUs (12 K rays: 150 us, 159 in units of 16; 49 K rays:
 // no difference, at four times the waves).
@@ -1846,6 +1857,7 @@ int enqueue_relaid(void (*kernel)(RelaidParams), RelaidParams P, int variant, si
     P.n_units = (P.n_rays + P.unit_rays - 1u) / P.unit_rays;
     int64_t blocks = (static_cast<int64_t>(P.n_chunks) + waves_per_block - 1) / waves_per_block;
     if (blocks > grid_blocks) blocks = grid_blocks;
+    if (threads == kWideThreads && P.n_rays < kOnePerCuRays && blocks > grid_blocks / 2) blocks = grid_blocks / 2;
     if (blocks < 1) blocks = 1;
     if (waves) *waves = static_cast<uint32_t>(blocks) * static_cast<uint32_t>(waves_per_block);
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(threads), lds, stream, P);
@@ -1908,7 +1920,8 @@ int launch_relaid(RelaidParams P, hipStream_t stream, uint32_t* scratch_queue = 
     navi_launch_info info = {};
     info.n_rays = P.n_rays;
     P.small_tables = (static_cast<uint64_t>(P.n_scenes) << (3u * P.cell_depth + 3u)) < (1ull << 32) ? 1u : 0u;
-    if (P.n_rays < kQuadMaxRays && P.n_rays < g_wide_min_rays.load(std::memory_order_relaxed)) {
+    const uint64_t wide_min = g_wide_min_rays.load(std::memory_order_relaxed);
+    if (P.n_rays < (wide_min == kWideMinRays ? kQuadMaxRays : std::min<uint64_t>(wide_min, kFastMinRays))) {
         info.pair = -1;
         const int code = launch_quad(P, stream, info);
         g_last_launch = info;

@@ -63,7 +63,7 @@ def wide_plane_depth(n_scenes: int, table_depth: int) -> int:
     ``plane_depth_wide``): the deepest P in [max(4, D - 2), min(D + 2, 8)] whose planes
     and scene table fit ``WIDE_PLANE_LDS_BYTES``; 0 when none does (such launches take
     the 256-thread workgroups). Launches of fewer rays than ``navi_set_wide_min_rays``
-    (default 2^19) take the 256-thread workgroups whatever this says."""
+    (default 2^19), and at its default launches below 851,968 rays, do not run on it."""
     for p in range(min(table_depth + 2, 8), max(4, table_depth - 2) - 1, -1):
         if n_scenes * (32 + _plane_bytes(p)) <= WIDE_PLANE_LDS_BYTES:
             return p
