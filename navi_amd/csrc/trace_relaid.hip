@@ -8,8 +8,8 @@
 //     (trace_quad.hpp); the rest below is about the larger ones;
 //   * two kernels: the fast march (monotone, tame, shallow scenes with split
 //     planes, the library compiler's) alone in trace_fast_kernel at eight
-//     waves per SIMD, in two 1024-thread workgroups per CU for launches of at
-//     least 2^19 rays (planes up to two levels below the cell table) or eight
+//     waves per SIMD, in two 1024-thread workgroups per CU (one below
+//     kOnePerCuRays; planes up to two levels below the cell table) or eight
 //     256-thread ones, everything in trace_relaid_kernel at seven; a launch
 //     enqueues the first when its planes fit, the second after it (returning
 //     at once when the first traced the launch), see launch_relaid;
@@ -138,6 +138,7 @@ struct RelaidParams {
     uint32_t n_chunks;
     uint32_t* __restrict__ queue;  // [next unit, finished waves], or null: static schedule
     uint32_t n_units;              // work units of unit_rays rays
+    uint32_t taper_from;           // first unit after which half of the fast kernel's waves claim no more
     uint32_t unit_rays;            // 128 (2 tiles), or 64 for batches too small to fill the chip
     uint32_t small_tables;         // the cell tables span fewer than 2^32 bytes
     uint32_t dist_dtype;           // NAVI_DIST_*: out_d holds float, bfloat16 or float16
@@ -319,6 +320,15 @@ constexpr uint32_t kQuadMaxRays = 13u << 16;
 // 719 and 687, 472 and 541, 452 and 541; 3.1 M: 1164 and 1031, 1155 and 993, 738 and 813,
 // 729 and 821.
 constexpr uint32_t kOnePerCuRays = 5u << 18;
+// Larger wide launches let every SIMD's waves thin out before the queue runs dry: with
+// so many rays left to claim, every second four waves of a workgroup (one per SIMD)
+// finish what they hold and claim no more. Us at 1.57 M rays, thinned out with 0, 0.52 M,
+// 0.79 M and 1.05 M rays left: 16 1024^3 scenes 763, 731, 717, 699, a 512^3 room grid 687,
+// 677, 663, 669, a 256^3 volume 541, 506, 495, 498; at 3.1 M 1051, 1009, 1012, 994 and 981,
+// 978, 990, 990 and 814, 781, 768, 770; at 12.6 M 2447, 2431, 2430, 2431 and 2694, 2684,
+// 2690, 2693.
+constexpr uint32_t kTaperRays = 3u << 18;
+static_assert(kTaperRays < kOnePerCuRays, "a tapered launch has more rays");
 // ... and the smallest of those in units of 4 rays, which wait less on each
 // other and reach more CUs (12 K rays: 150 us, 159 in units of 16; 49 K rays:
 // no difference, at four times the waves).
@@ -420,6 +430,7 @@ __device__ __forceinline__ uint32_t plane_cell(float p, float off, float scale, 
 struct Sched {
     uint32_t wave, n_waves, seq_end, seq_next, unit, unit_used;
     bool exhausted;
+    bool last;  // the wave claims no unit after the one it holds
 };
 
 __device__ __forceinline__ Sched sched_init(const RelaidParams& P) {
@@ -431,6 +442,7 @@ __device__ __forceinline__ Sched sched_init(const RelaidParams& P) {
     S.seq_next = 0;
     S.unit = 0;
     S.unit_used = P.unit_rays;
+    S.last = false;
     S.exhausted = (P.queue == nullptr) ? (S.seq_end == 0) : false;
     return S;
 }
@@ -450,10 +462,13 @@ __device__ __forceinline__ uint32_t claim(const RelaidParams& P, Sched& S, uint3
         const uint32_t avail = P.unit_rays - S.unit_used;
         if (rank < avail) q = S.unit * P.unit_rays + S.unit_used + rank;
         if (n_need > avail) {
-            uint32_t claimed = 0;
-            if (lane == 0) claimed = atomicAdd(P.queue, 1u);
-            claimed = __builtin_amdgcn_readlane(claimed, 0);
+            uint32_t claimed = P.n_units;
+            if (!S.last) {
+                if (lane == 0) claimed = atomicAdd(P.queue, 1u);
+                claimed = __builtin_amdgcn_readlane(claimed, 0);
+            }
             if (claimed < P.n_units) {
+                if (kQueued) S.last = (S.wave & 4u) != 0u && claimed >= P.taper_from;
                 if (rank >= avail) q = claimed * P.unit_rays + (rank - avail);
                 S.unit = claimed;
                 S.unit_used = n_need - avail;
@@ -1857,7 +1872,12 @@ int enqueue_relaid(void (*kernel)(RelaidParams), RelaidParams P, int variant, si
     P.n_units = (P.n_rays + P.unit_rays - 1u) / P.unit_rays;
     int64_t blocks = (static_cast<int64_t>(P.n_chunks) + waves_per_block - 1) / waves_per_block;
     if (blocks > grid_blocks) blocks = grid_blocks;
-    if (threads == kWideThreads && P.n_rays < kOnePerCuRays && blocks > grid_blocks / 2) blocks = grid_blocks / 2;
+    P.taper_from = P.n_units;
+    if (threads == kWideThreads && P.n_rays < kOnePerCuRays) {
+        if (blocks > grid_blocks / 2) blocks = grid_blocks / 2;
+    } else if (threads == kWideThreads) {
+        P.taper_from = P.n_units - kTaperRays / P.unit_rays;
+    }
     if (blocks < 1) blocks = 1;
     if (waves) *waves = static_cast<uint32_t>(blocks) * static_cast<uint32_t>(waves_per_block);
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(threads), lds, stream, P);

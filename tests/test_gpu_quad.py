@@ -66,3 +66,20 @@ def test_last_rays_of_a_wave_match_the_oracle(resident, corpus, envs, az, el, bi
         _native.set_wide_min_rays(prev)
     assert info["fast_wide"] and not info["quad"] and info["fast_planes"] == 8, info
     _compare(got, ref, 30.0, f"{envs}x{az}x{el}/{bins}/{steps}")
+
+
+@pytest.mark.parametrize("envs", [103, 104, 159, 160])
+def test_launch_shapes_of_mid_size_batches(resident, corpus, envs):  # noqa: F811
+    """8192 rays an env on both sides of the lines between four lanes per ray and one
+    (851,968 rays), and between one workgroup per CU and two whose waves thin out
+    towards the end (1,310,720)."""
+    from navi_amd import _native
+
+    env_scene, o, d = _rays(corpus, envs, 128, 64, seed=envs)
+    ref = _oracle_multi([c.words for c in corpus], [c.bbox_min_list + c.bbox_max for c in corpus],
+                        env_scene.astype(np.int32), o, d, 160, 30.0)
+    got = _run(resident, env_scene, o, d, 160, 30.0, elevation_bins=64)
+    info = _native.last_launch()
+    # 256 CUs of 16 or 32 waves
+    assert info["quad"] == (envs < 104) and (info["quad"] or info["waves"] == (4096 if envs < 160 else 8192)), info
+    _compare(got, ref, 30.0, str(envs))
