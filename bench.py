@@ -261,7 +261,7 @@ def summarize_profiles(root: Path, out_path: Path) -> None:
         times: dict = {}
         for r in kt:
             times.setdefault(r["Kernel_Name"], []).append((int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e6)
-        tracers = [k for k in times if ("trace_fast_kernel" in k or "trace_relaid_kernel" in k)]
+        tracers = [k for k in times if any(t in k for t in ("trace_fast_kernel", "trace_relaid_kernel", "trace_quad_kernel"))]
         kernels = [max(tracers, key=lambda k: sum(times[k]))] if tracers else []
         kernels += [k for k in times if "observation_kernel" in k]
         fetch, write, sq = per_dispatch(wdir / "fetch"), per_dispatch(wdir / "write"), per_dispatch(wdir / "sq")
