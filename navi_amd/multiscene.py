@@ -85,6 +85,14 @@ def default_table_depth(n_scenes: int) -> int:
     return 4
 
 
+def _flat_words(words: torch.Tensor) -> torch.Tensor:
+    """A tensor of DAG words as the conversion kernels read them, one after another from its
+    first: a strided or expanded tensor (which ``reshape(-1)`` returns as it is) is copied."""
+    if words.dtype not in (torch.int64, torch.uint64):
+        raise TypeError(f"a tensor of DAG words must be int64, not {words.dtype}")
+    return words.detach().view(torch.int64).reshape(-1).contiguous()
+
+
 class ResidentScenes:
     """Concatenated word pool + scene table on one device.
 
@@ -108,7 +116,7 @@ class ResidentScenes:
         chunks = []  # uint64 arrays, or int64 tensors that are already on the device
         for i, (words, lo, hi) in enumerate(scenes):
             if isinstance(words, torch.Tensor) and words.device == self.device and words.is_cuda:
-                w = words.detach().view(torch.int64).reshape(-1)
+                w = _flat_words(words)
                 size = int(w.numel())
             else:
                 w = np.ascontiguousarray(np.asarray(words).view(np.uint64).reshape(-1))

@@ -97,6 +97,26 @@ def test_compiled_scenes(depth, monkeypatch):
     _compare(scenes, monkeypatch, True, table_depth=depth)
 
 
+@pytest.mark.parametrize("keep_words", [False, True])
+def test_device_words_of_any_stride(keep_words):
+    """Words that lie apart in their tensor, or are one word expanded, convert as their
+    copies do."""
+    scene = S.box_room(seed=1, resolution=64)
+    scene.compile(threads=8)
+    plain = torch.from_numpy(scene.words.view(np.int64)).cuda()
+    apart = torch.full((plain.numel(), 3), -1, dtype=torch.int64, device="cuda")
+    apart[:, 1] = plain
+    node = torch.tensor([_node(0, 1)], dtype=torch.int64, device="cuda")
+    for words, copy in ((apart[:, 1], plain), (node.expand(5), node.repeat(5))):
+        assert not words.is_contiguous()
+        got, want = (ResidentScenes([(w, scene.bbox_min_list, scene.bbox_max)], "cuda", keep_words=keep_words)
+                     for w in (words, copy))
+        assert got.n_records == want.n_records
+        for name in ("records", "cell_tables", "relaid_table", "pool"):
+            a, b = getattr(got, name), getattr(want, name)
+            assert (a is None) == (b is None) and (a is None or torch.equal(a, b)), name
+
+
 def test_refused_while_capturing():
     """The conversion waits for its stream, so a capturing stream is an error that leaves
     the capture as it is."""
