@@ -177,7 +177,11 @@ class ResidentScenes:
 
     @staticmethod
     def _words(chunk: Any) -> torch.Tensor:
-        return chunk if isinstance(chunk, torch.Tensor) else torch.from_numpy(chunk.view(np.int64))
+        if isinstance(chunk, torch.Tensor):
+            return chunk
+        # (a frozen or memory-mapped file's array is copied: torch warns of tensors over memory
+        # that must not be written)
+        return torch.from_numpy((chunk if chunk.flags.writeable else chunk.copy()).view(np.int64))
 
     def _table_depth_for(self, rtable: np.ndarray, table_depth: int | None) -> int:
         if table_depth is not None:

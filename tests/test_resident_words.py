@@ -1,6 +1,8 @@
 """The DAG words that ``ResidentScenes`` takes, on the CPU: what the conversion kernels, which
 read consecutive words from a pointer, are given."""
 
+import warnings
+
 import numpy as np
 import pytest
 import torch
@@ -36,3 +38,26 @@ def test_tensor_words_are_consecutive(name):
 def test_other_types_are_refused(dtype):
     with pytest.raises(TypeError, match="int64"):
         multiscene._flat_words(torch.zeros(8, dtype=dtype))
+
+
+@pytest.mark.parametrize("keep_words", [False, True])
+@pytest.mark.parametrize("source", ["frozen", "mapped", "bytes"])
+def test_read_only_words_load_without_a_warning(source, keep_words, tmp_path):
+    """Words of a frozen array, a memory-mapped file and a byte string, as an asset's reader
+    holds them."""
+    words = np.array([0xFF << 55 | 1, *[9] * 8, 1 << 63 | 3 << 16 | 0x2E66], np.uint64)
+    if source == "mapped":
+        words.tofile(tmp_path / "words")
+        given = np.memmap(tmp_path / "words", np.uint64, "r")
+    else:
+        given = np.frombuffer(words.tobytes(), np.uint64)
+        if source == "frozen":
+            given = words.copy()
+            given.setflags(write=False)
+    assert not given.flags.writeable
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        got = multiscene.ResidentScenes([(given, [0.0] * 3, [1.0] * 3)], "cpu", keep_words=keep_words)
+        upload = got._words(got.pool if keep_words else np.ascontiguousarray(given))
+    assert got.relaid_ok and got.word_counts == [10]
+    assert np.array_equal(upload.numpy().view(np.uint64), words)
