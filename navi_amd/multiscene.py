@@ -143,11 +143,10 @@ class ResidentScenes:
                 self.pool[int(at):int(at) + n] = self._words(w)
         self.table = torch.from_numpy(table.view(np.uint8).copy()).to(self.device)
 
-        # device record layout (one 32-byte record per internal node), made on the
-        # device where its conversion covers every scene, else on the host
+        # device record layout (one 32-byte record per internal node)
         self.n_leaves = 0
         self.leaves = None
-        self.relaid_ok = self._layout_on_device(chunks, table_depth) or self._layout_on_host(chunks, table_depth)
+        self.relaid_ok = self._layout(chunks, table_depth)
         self._order_key = None
         self._order = None
         # scene order by measured cost (module docstring)
@@ -191,107 +190,106 @@ class ResidentScenes:
         deepest = max(int(d) for d in rtable["max_depth"])  # 0xffffffff for a cycle
         return max(4, min(default_table_depth(self.n_scenes), deepest + 1))
 
-    def _new_rtable(self) -> np.ndarray:
+    def _layout(self, chunks: list, table_depth: int | None) -> bool:
+        """The record layout of the scenes: records (child records as pool indices), cell
+        tables, leaf table, scene table. Each scene's records are converted on the device,
+        or on the host where the device does not cover it; both give the same arrays. False
+        when the record layout cannot hold the scenes. Waits for the device: the arrays are
+        complete for every stream when it returns."""
         rtable = np.zeros(self.n_scenes, dtype=_native.RELAID_SCENE_DTYPE)
         rtable["bbox_min"] = self.host_table["bbox_min"]
         rtable["bbox_max"] = self.host_table["bbox_max"]
-        return rtable
-
-    def _layout_on_device(self, chunks: list, table_depth: int | None) -> bool:
-        """Records and cell tables converted on the device (``navi_relayout_device``), the
-        same arrays as the host's; False when it leaves a scene to the host. Waits for the
-        device: the arrays are complete for every stream when it returns."""
-        if self.device.type != "cuda":
-            return False
-        lib = _native.lib()
-        rtable = self._new_rtable()
-        pools = []
-        offset = 0
-        with torch.cuda.device(self.device):
-            current = torch.cuda.current_stream(self.device)
-            stream = current.cuda_stream
-            state = torch.empty(_native.RELAYOUT_STATE_WORDS, dtype=torch.int32, device=self.device)
-            for i, chunk in enumerate(chunks):
-                n, at = self.word_counts[i], int(self.host_table[i]["word_offset"])
-                words = self.pool[at:at + n] if self.pool is not None else self._words(chunk).to(self.device)
-                mark, order = (torch.empty(n, dtype=torch.int32, device=self.device) for _ in range(2))
-                layout = _native.DeviceLayout()
-                _native.check(lib.navi_relayout_device(words.data_ptr(), n, mark.data_ptr(), order.data_ptr(),
-                                                       state.data_ptr(), ctypes.byref(layout), stream))
-                # a pool holds fewer than 2^27 records (_layout_on_host)
-                if not layout.converted or offset + layout.n_records >= (1 << 27):
-                    return False
-                records = torch.empty(8 * layout.n_records, dtype=torch.int32, device=self.device)
-                _native.check(lib.navi_relayout_device_records(words.data_ptr(), n, mark.data_ptr(), order.data_ptr(),
-                                                               layout.n_records, offset, records.data_ptr(), stream))
-                pools.append(records)
-                rtable[i]["rec_offset"] = rtable[i]["root_slot"] = offset
-                rtable[i]["n_records"] = layout.n_records
-                rtable[i]["max_depth"] = layout.max_depth
-                rtable[i]["flags"] = layout.flags
-                offset += layout.n_records
-            self.table_depth = self._table_depth_for(rtable, table_depth)
-            self.records = torch.cat(pools) if len(pools) > 1 else pools[0]
-            self.n_records = offset
-            cells = 8 ** self.table_depth
-            self.cell_tables = torch.empty(self.n_scenes * cells, dtype=torch.int64, device=self.device)
-            for i in range(self.n_scenes):
-                _native.check(lib.navi_build_cell_table_device(
-                    self.records.data_ptr(), self.n_records, int(rtable[i]["root_slot"]), self.table_depth,
-                    self.cell_tables.data_ptr() + 8 * cells * i, stream))
-            self.relaid_table = torch.from_numpy(rtable.view(np.uint8).copy()).to(self.device)
-            self.record_counts = [int(c) for c in rtable["n_records"]]
-            current.synchronize()
-        return True
-
-    def _layout_on_host(self, chunks: list, table_depth: int | None) -> bool:
-        """Records and cell tables converted on the host and uploaded; leaves of semantic
-        0x7fff or above go to one leaf table shared by the pool. False when the record
-        layout cannot hold the scenes."""
-        rtable = self._new_rtable()
-        recs = []
+        recs = []  # uint32 arrays of the host's, or int32 tensors on the device
         leaf_tables = []
-        roff = 0
-        loff = 0
+        offset = n_leaves = 0
         for i, chunk in enumerate(chunks):
-            w = chunk.cpu().numpy().view(np.uint64) if isinstance(chunk, torch.Tensor) else chunk
-            try:
-                rec, root, _levels, leaves = _native.relayout_leaves(w)
-                rec, root = _native.rebase_leaves(rec, root, loff)
-            except RuntimeError:
+            converted = (self._layout_on_device(rtable[i], i, chunk, offset)
+                         or self._layout_on_host(rtable[i], chunk, offset, n_leaves))
+            if not converted:
                 return False
-            leaf_tables.append(leaves)
-            loff += int(leaves.size)
-            rtable[i]["rec_offset"] = roff
-            rtable[i]["n_records"] = rec.shape[0]
-            # child record slots become absolute pool indices
-            rec = rec.copy()
-            child = rec < 0x7FFFFFFD
-            rec[child] += np.uint32(roff)
-            rtable[i]["root_slot"] = root if root & 0x80000000 else roff + root
-            recs.append(rec)
-            roff += rec.shape[0]
-        # navi_trace_relaid reads the pool through a buffer resource whose
-        # 32-bit byte size must not wrap: fewer than 2^27 records
-        if roff >= (1 << 27):
-            return False
-        allrec = np.concatenate(recs) if roff else np.zeros((1, 8), np.uint32)
-        all_leaves = np.concatenate(leaf_tables) if loff else np.zeros(0, np.uint32)
-        for i in range(self.n_scenes):
-            rtable[i]["max_depth"] = _native.record_depth(allrec[:roff], int(rtable[i]["root_slot"]))
-            rtable[i]["flags"] = _native.scene_flags(allrec[:roff], int(rtable[i]["root_slot"]), all_leaves)
-        if loff:
-            self.n_leaves = loff
-            self.leaves = torch.from_numpy(all_leaves.view(np.int32).copy()).to(self.device)
+            records, leaves = converted
+            recs.append(records)
+            offset += int(rtable[i]["n_records"])
+            if leaves is not None and leaves.size:
+                leaf_tables.append(leaves)
+                n_leaves += int(leaves.size)
+            # navi_trace_relaid reads the pool through a buffer resource whose
+            # 32-bit byte size must not wrap: fewer than 2^27 records
+            if offset >= (1 << 27):
+                return False
+        self.n_records = offset
+        self.record_counts = [int(c) for c in rtable["n_records"]]
+        if n_leaves:
+            self.n_leaves = n_leaves
+            self.leaves = torch.from_numpy(np.concatenate(leaf_tables).view(np.int32)).to(self.device)
         self.table_depth = self._table_depth_for(rtable, table_depth)
-        tables = np.concatenate([_native.cell_table(allrec[:roff], int(rtable[i]["root_slot"]), self.table_depth)
-                                 for i in range(self.n_scenes)])
-        self.cell_tables = torch.from_numpy(tables.view(np.int64)).to(self.device)
-        self.n_records = int(roff)
-        self.records = torch.from_numpy(allrec.view(np.int32).reshape(-1).copy()).to(self.device)
+        if all(isinstance(r, np.ndarray) for r in recs):
+            allrec = np.concatenate(recs) if offset else np.zeros(8, np.uint32)
+            self.records = torch.from_numpy(allrec.view(np.int32)).to(self.device)
+        else:
+            self.records = torch.cat([r if isinstance(r, torch.Tensor) else
+                                      torch.from_numpy(r.view(np.int32)).to(self.device) for r in recs])
+        cells = 8 ** self.table_depth
+        roots = [int(r) for r in rtable["root_slot"]]
+        if self.device.type == "cuda":
+            self.cell_tables = torch.empty(self.n_scenes * cells, dtype=torch.int64, device=self.device)
+            with torch.cuda.device(self.device):
+                current = torch.cuda.current_stream(self.device)
+                for i, root in enumerate(roots):
+                    _native.check(_native.lib().navi_build_cell_table_device(
+                        self.records.data_ptr(), self.n_records, root, self.table_depth,
+                        self.cell_tables.data_ptr() + 8 * cells * i, current.cuda_stream))
+                current.synchronize()
+        else:
+            tables = np.concatenate([_native.cell_table(allrec[:8 * offset], root, self.table_depth)
+                                     for root in roots])
+            self.cell_tables = torch.from_numpy(tables.view(np.int64))
         self.relaid_table = torch.from_numpy(rtable.view(np.uint8).copy()).to(self.device)
-        self.record_counts = [int(r.shape[0]) for r in recs]
         return True
+
+    def _layout_on_device(self, entry: Any, i: int, chunk: Any, offset: int) -> tuple[Any, Any] | None:
+        """Scene ``i``'s records, the pool's from ``offset`` on, converted on the device
+        (``navi_relayout_device``) and its ``entry`` of the scene table; None when that leaves
+        the scene to the host."""
+        if self.device.type != "cuda":
+            return None
+        lib = _native.lib()
+        with torch.cuda.device(self.device):
+            stream = torch.cuda.current_stream(self.device).cuda_stream
+            state = torch.empty(_native.RELAYOUT_STATE_WORDS, dtype=torch.int32, device=self.device)
+            n, at = self.word_counts[i], int(self.host_table[i]["word_offset"])
+            words = self.pool[at:at + n] if self.pool is not None else self._words(chunk).to(self.device)
+            mark, order = (torch.empty(n, dtype=torch.int32, device=self.device) for _ in range(2))
+            layout = _native.DeviceLayout()
+            _native.check(lib.navi_relayout_device(words.data_ptr(), n, mark.data_ptr(), order.data_ptr(),
+                                                   state.data_ptr(), ctypes.byref(layout), stream))
+            if not layout.converted:
+                return None
+            records = torch.empty(8 * layout.n_records, dtype=torch.int32, device=self.device)
+            _native.check(lib.navi_relayout_device_records(words.data_ptr(), n, mark.data_ptr(), order.data_ptr(),
+                                                           layout.n_records, offset, records.data_ptr(), stream))
+        entry["rec_offset"] = entry["root_slot"] = offset
+        entry["n_records"], entry["max_depth"], entry["flags"] = layout.n_records, layout.max_depth, layout.flags
+        return records, None
+
+    @staticmethod
+    def _layout_on_host(entry: Any, chunk: Any, offset: int, leaf_offset: int) -> tuple[Any, Any] | None:
+        """A scene's records, the pool's from ``offset`` on, converted on the host, its leaves
+        of semantic 0x7fff or above (the pool's leaf table from ``leaf_offset`` on) and its
+        ``entry`` of the scene table; None when the record layout cannot hold it."""
+        w = chunk.cpu().numpy().view(np.uint64) if isinstance(chunk, torch.Tensor) else chunk
+        try:
+            rec, root, _levels, leaves = _native.relayout_leaves(w)
+            entry["max_depth"] = _native.record_depth(rec, root)
+            entry["flags"] = _native.scene_flags(rec, root, leaves)
+            rec, root = _native.rebase_leaves(rec, root, leaf_offset)
+        except RuntimeError:
+            return None
+        # child record slots become absolute pool indices
+        rec[rec < 0x7FFFFFFD] += np.uint32(offset)
+        entry["rec_offset"], entry["n_records"] = offset, rec.shape[0]
+        entry["root_slot"] = root if root & 0x80000000 else offset + root
+        return rec.reshape(-1), leaves
 
     @property
     def pool_bytes(self) -> int:

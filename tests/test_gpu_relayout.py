@@ -97,6 +97,32 @@ def test_compiled_scenes(depth, monkeypatch):
     _compare(scenes, monkeypatch, True, table_depth=depth)
 
 
+@pytest.mark.parametrize("names", [("table_leaf", "room", "shared", "room"), ("room", "one_leaf", "two_depths", "room"),
+                                   ("one_record", "table_leaf", "room", "table_leaf_high"), ("one_leaf", "one_leaf"),
+                                   ("cycle", "table_leaf_high")])
+def test_pools_of_both_conversions(names, monkeypatch):
+    """A pool whose scenes are covered by the device, left to the host, or both: the same
+    arrays as an all-host pool, and the host converts only what is left to it."""
+    room = S.box_room(seed=1, resolution=64)
+    room.compile(threads=8)
+    dags = {k: np.array(w, np.uint64) for k, w in _hand_made().items()} | {"room": room.words}
+    scenes = [(dags[name], [0.0] * 3, [1.0 + k] * 3) for k, name in enumerate(names)]
+    want = ResidentScenes(scenes, "cpu")
+    host = ResidentScenes._layout_on_host
+    converted = []
+    monkeypatch.setattr(ResidentScenes, "_layout_on_host",
+                        lambda self, entry, chunk, *a: converted.append(1) or host(entry, chunk, *a))
+    for keep_words in (False, True):
+        converted.clear()
+        got = ResidentScenes(scenes, "cuda", keep_words=keep_words)
+        assert len(converted) == sum(name in HOST_ONLY for name in names)
+        assert got.relaid_ok and got.n_records == want.n_records and got.n_leaves == want.n_leaves
+        assert got.record_counts == want.record_counts and got.table_depth == want.table_depth
+        for name in ("records", "cell_tables", "relaid_table", "table", "leaves"):
+            a, b = getattr(got, name), getattr(want, name)
+            assert (a is None) == (b is None) and (a is None or torch.equal(a.cpu(), b)), name
+
+
 @pytest.mark.parametrize("keep_words", [False, True])
 def test_device_words_of_any_stride(keep_words):
     """Words that lie apart in their tensor, or are one word expanded, convert as their
