@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from navi_amd import _native
+from navi_amd import _native, multiscene
 from navi_amd import scenes as S
 from navi_amd.multiscene import ResidentScenes
 
@@ -62,6 +62,7 @@ HOST_ONLY = ("levels_32", "one_leaf", "table_leaf", "table_leaf_high", "cycle", 
 
 def _compare(scenes, monkeypatch, on_device, **kw):
     want = ResidentScenes(scenes, "cpu", **kw)
+    monkeypatch.setattr(multiscene, "DEVICE_MIN_WORDS", 0)
     if on_device:
         def refuse(self, *a):
             raise AssertionError("converted on the host")
@@ -108,6 +109,7 @@ def test_pools_of_both_conversions(names, monkeypatch):
     dags = {k: np.array(w, np.uint64) for k, w in _hand_made().items()} | {"room": room.words}
     scenes = [(dags[name], [0.0] * 3, [1.0 + k] * 3) for k, name in enumerate(names)]
     want = ResidentScenes(scenes, "cpu")
+    monkeypatch.setattr(multiscene, "DEVICE_MIN_WORDS", 0)
     host = ResidentScenes._layout_on_host
     converted = []
     monkeypatch.setattr(ResidentScenes, "_layout_on_host",
@@ -123,10 +125,26 @@ def test_pools_of_both_conversions(names, monkeypatch):
             assert (a is None) == (b is None) and (a is None or torch.equal(a.cpu(), b)), name
 
 
+@pytest.mark.parametrize("n,on_host", [(1, True), ((1 << 14) - 1, True), (1 << 14, False)])
+def test_small_scenes_are_converted_on_the_host(n, on_host, monkeypatch):
+    host = ResidentScenes._layout_on_host
+    converted = []
+    monkeypatch.setattr(ResidentScenes, "_layout_on_host",
+                        lambda self, entry, chunk, *a: converted.append(1) or host(entry, chunk, *a))
+    words = np.zeros(n, np.uint64)
+    words[0] = _node(0, 1)
+    for source in (words, torch.from_numpy(words.view(np.int64)).cuda()):
+        converted.clear()
+        got = ResidentScenes([(source, [0.0] * 3, [1.0] * 3)], "cuda")
+        assert bool(converted) == on_host and got.n_records == 1
+        assert bool((got.records.cpu() == 0x7FFFFFFF).all())
+
+
 @pytest.mark.parametrize("keep_words", [False, True])
-def test_device_words_of_any_stride(keep_words):
+def test_device_words_of_any_stride(keep_words, monkeypatch):
     """Words that lie apart in their tensor, or are one word expanded, convert as their
     copies do."""
+    monkeypatch.setattr(multiscene, "DEVICE_MIN_WORDS", 0)
     scene = S.box_room(seed=1, resolution=64)
     scene.compile(threads=8)
     plain = torch.from_numpy(scene.words.view(np.int64)).cuda()
