@@ -353,6 +353,10 @@ int navi_trace_relaid_poses(const uint32_t* records, uint64_t n_records, const n
 #define NAVI_DIST_BF16 1  /* bfloat16 (uint16 storage) */
 #define NAVI_DIST_F16 2   /* IEEE binary16 */
 
+/* navi_relaid_launch.scene_hints: what the caller knows of the scene table, for
+ * the launch shape (results are the same with or without). */
+#define NAVI_SCENES_FAST 1u /* every scene has NAVI_SCENE_NONNEG_LEAVES and max_depth <= 30 */
+
 /* Arguments of navi_trace_relaid_ex (device pointers unless noted). */
 typedef struct navi_relaid_launch {
     const uint32_t* records;           /* record pool, as navi_trace_relaid */
@@ -361,6 +365,7 @@ typedef struct navi_relaid_launch {
     uint32_t n_leaves;                 /* its entries (0 for none) */
     const navi_relaid_scene* scenes;
     int32_t n_scenes;
+    uint32_t scene_hints;              /* NAVI_SCENES_* (0: nothing known) */
     const uint64_t* cell_tables;
     int32_t table_depth;
     const int32_t* env_scene;          /* [n_envs] or NULL (scene 0) */
@@ -394,11 +399,13 @@ int navi_trace_relaid_ex(const navi_relaid_launch* launch, void* stream);
  * Launch shape of the record-layout tracer (no reference counterpart: a tuning
  * knob of this library). Launches of at least `n_rays` rays whose scenes'
  * split planes fit two levels below the cell tables in 80 KiB of LDS run in
- * 1024-thread workgroups, a lane per ray; smaller launches below 2^19 rays run
- * with four lanes per ray (trace_quad_kernel), smaller launches of 2^19 rays and
- * more in 256-thread workgroups. At the default threshold launches below 851,968
- * rays run with four lanes per ray. Results are identical either way. Process-wide, thread-safe; takes effect from the next launch. Returns
- * the previous value (default 2^19).
+ * 1024-thread workgroups, a lane per ray; smaller launches below 2^19 rays that
+ * suit it run with four lanes per ray (trace_quad_kernel), others in 256-thread
+ * workgroups. At the default threshold launches of up to 851,968 rays that suit it
+ * (a fine sensor's angular tiles; fewer in other orders, in envs of few rays,
+ * without NAVI_SCENES_FAST or over 1000 m) run with four lanes per ray. Results are
+ * identical either way. Process-wide, thread-safe; takes effect from the next
+ * launch. Returns the previous value (default 2^19).
  */
 uint64_t navi_set_wide_min_rays(uint64_t n_rays);
 

@@ -127,12 +127,13 @@ class RelaidLaunch(ctypes.Structure):
     """navi_relaid_launch (include/navi_trace.h)."""
 
     _fields_ = [("records", _vp), ("n_records", ctypes.c_uint64), ("leaves", _vp), ("n_leaves", ctypes.c_uint32),
-                ("scenes", _vp), ("n_scenes", ctypes.c_int32), ("cell_tables", _vp), ("table_depth", ctypes.c_int32),
-                ("env_scene", _vp), ("env_order", _vp), ("n_envs", ctypes.c_int64), ("rays_per_env", ctypes.c_int64),
-                ("elevation_bins", ctypes.c_int32), ("origins", _vp), ("dirs", _vp), ("local_dirs", _vp),
-                ("env_pos", _vp), ("env_rot", _vp), ("out_distances", _vp), ("out_semantics", _vp),
-                ("out_steps", _vp), ("max_steps", ctypes.c_int32), ("max_distance", ctypes.c_float),
-                ("hit_epsilon", ctypes.c_float), ("distance_dtype", ctypes.c_int32)]
+                ("scenes", _vp), ("n_scenes", ctypes.c_int32), ("scene_hints", ctypes.c_uint32),
+                ("cell_tables", _vp), ("table_depth", ctypes.c_int32), ("env_scene", _vp), ("env_order", _vp),
+                ("n_envs", ctypes.c_int64), ("rays_per_env", ctypes.c_int64), ("elevation_bins", ctypes.c_int32),
+                ("origins", _vp), ("dirs", _vp), ("local_dirs", _vp), ("env_pos", _vp), ("env_rot", _vp),
+                ("out_distances", _vp), ("out_semantics", _vp), ("out_steps", _vp), ("max_steps", ctypes.c_int32),
+                ("max_distance", ctypes.c_float), ("hit_epsilon", ctypes.c_float),
+                ("distance_dtype", ctypes.c_int32)]
 
 
 class LaunchInfo(ctypes.Structure):
@@ -194,6 +195,7 @@ RELAID_SCENE_DTYPE = [("rec_offset", "<u8"), ("n_records", "<u4"), ("root_slot",
                       ("bbox_min", "<f4", (3,)), ("bbox_max", "<f4", (3,)), ("max_depth", "<u4"),
                       ("flags", "<u4")]
 SCENE_NONNEG_LEAVES = 1  # navi_relaid_scene.flags bit (include/navi_trace.h)
+SCENES_FAST = 1  # navi_relaid_launch.scene_hints bit
 DIST_F32, DIST_BF16, DIST_F16 = 0, 1, 2  # navi_relaid_launch.distance_dtype
 
 

@@ -4,8 +4,8 @@
 // checkout); tests compare both against the CPU oracle bit for bit.
 //
 // Execution model (CDNA4, wave64):
-//   * launches below kQuadMaxRays rays: trace_quad_kernel, four lanes per ray
-//     (trace_quad.hpp); the rest below is about the larger ones;
+//   * launches of few units of rays (quads_pay): trace_quad_kernel, four lanes per
+//     ray (trace_quad.hpp); the rest below is about the larger ones;
 //   * two kernels: the fast march (monotone, tame, shallow scenes with split
 //     planes, the library compiler's) alone in trace_fast_kernel at eight
 //     waves per SIMD, in two 1024-thread workgroups per CU (one below
@@ -293,7 +293,7 @@ constexpr size_t kFastLds = 20480;
 constexpr int kWideThreads = 1024;
 constexpr size_t kFastLdsWide = 81920;
 // Launches of at least so many rays run wide where trace_quad_kernel does not take
-// them (kQuadMaxRays); with the threshold raised (navi_set_wide_min_rays), launches
+// them; with the threshold raised (navi_set_wide_min_rays), launches
 // below it take the 256-thread workgroups from kFastMinRays rays on, which spread
 // a batch over more CUs (786 K rays on one 512^3 scene 3% faster wide).
 constexpr uint64_t kWideMinRays = 1u << 19;
@@ -302,16 +302,44 @@ std::atomic<uint64_t> g_wide_min_rays{kWideMinRays};
 // threshold whose planes do not fit): the combined kernel alone saves the
 // second launch.
 constexpr uint32_t kFastMinRays = 1u << 19;
-// Smaller launches take trace_quad_kernel, four lanes per ray (with the wide
-// threshold moved, those below it and below kFastMinRays): they last as long as
-// their longest rays' chains of steps, and a quad's step takes about two thirds of
-// the time (49 K rays on a 128^3 volume 112 -> 72 us, 12 K on a 512^3 room grid 243 ->
-// 150 us). From about a million rays on the work counts. Us in quads and a lane each
-// (the better of its two grids below): 836 K rays of 16 1024^3 scenes 524 and 570, of
-// a 512^3 room grid 538 and 517, of a 256^3 volume 355 and 325, of a 128^3 room 231
-// and 318; 688 K: 481 and 548, 459 and 475, 303 and 294, 205 and 295; 1.03 M: 637 and
-// 602, 610 and 572, 413 and 362, 283 and 346.
-constexpr uint32_t kQuadMaxRays = 13u << 16;
+// Launches of few units (of 16 rays, or 4) take trace_quad_kernel, four lanes per ray:
+// they last as long as their longest rays' chains of steps, and a quad's step takes about
+// two thirds of the time (49 K rays on a 128^3 volume 112 -> 72 us, 12 K on a 512^3 room
+// grid 243 -> 150 us). With more units the work counts, and a unit's idle lanes: those of
+// an env's last unit, and those of rays that end before the unit's longest (nothing is
+// refilled). So the line lies by units, and by what is known of them:
+// * angular tiles of a fine sensor (neighbours of much the same length): 53,248 units, 852 K
+//   rays. Us in quads and a lane each (the better of its two grids below): 836 K rays of 16
+//   1024^3 scenes 524 and 570, of a 512^3 room grid 538 and 517, of a 256^3 volume 355 and
+//   325, of a 128^3 room 231 and 318; 688 K: 481 and 548, 459 and 475, 303 and 294, 205 and
+//   295; 1.03 M: 637 and 602, 610 and 572, 413 and 362, 283 and 346.
+constexpr uint32_t kQuadTiledUnits = 13u << 12;
+constexpr uint32_t kQuadFineRays = 2048;  // rays of such a sensor
+// * other full units, rays in the sensor's order or in none, tiles of a coarse sensor:
+//   32,768 units, 524 K rays. The scenes differ by more than the sides here, so the line
+//   lies by their mean. In the sensor's order, quads, a lane each in one workgroup per CU
+//   and in two: 393 K rays of a 512^3 room grid 360, 362 and 446 us, of a 256^3 volume 223,
+//   256 and 338, of a 64^3 room 102, 195 and 245; 590 K 473, 425 and 545, 298, 294 and 403,
+//   147, 245 and 336. In no order 393 K 477, 352 and 450, 263, 253 and 344, 122, 195 and 245;
+//   590 K 658, 416 and 550, 348, 292 and 403, 172, 235 and 327. Tiles of 16 x 8, quads and a
+//   lane each in two: 390 K 399 and 364, 232 and 327, 122 and 241; 680 K 636 and 476, 349 and
+//   409, 196 and 354.
+constexpr uint32_t kQuadFullUnits = 1u << 15;
+// * units with idle lanes, and those of so few rays an env that neighbours have little in
+//   common: 8192 units, as many as the chip holds at once.
+//   Rays in random directions, quads and a lane each: 65 K rays of 1, 2, 8 and 17 an env
+//   (65,536, 32,768, 8192 and 7710 units) on a 512^3 room grid 469, 356, 212 and 243 us
+//   against 282, 281, 273 and 274; 131 K of 8, 17 and 33 an env (16,384, 15,420 and 11,916
+//   units) 330, 363 and 279 against 300, 293 and 290; 262 K of 48 an env (16,384 full units)
+//   392 against 367; 800 K of one an env 4360 against 714.
+constexpr uint32_t kQuadSparseUnits = 1u << 13;
+constexpr uint32_t kQuadEnvRays = 128;
+// * launches of the general march, whose step in quads is longer (ranges of 1000 and more,
+//   scenes not known to take the fast march): 4096 units, 65 K full ones' rays. Quads and a
+//   lane each on a 256^3 room grid: 4680 units 338 and 342 us, 8192 units of tiled rays 369
+//   and 378, of 8 rays an env 393 and 347, 12,288 of tiled rays 475 and 417, 30,720 783 and
+//   659.
+constexpr uint32_t kQuadGeneralUnits = 1u << 12;
 // Wide launches of fewer rays run one workgroup per CU instead of two: a SIMD that
 // issues for four waves takes half the time per step, which shortens the chains that
 // such a launch ends on, and its waves refill twice as often. Us with one and two
@@ -329,9 +357,10 @@ constexpr uint32_t kOnePerCuRays = 5u << 18;
 // 2690, 2693.
 constexpr uint32_t kTaperRays = 3u << 18;
 static_assert(kTaperRays < kOnePerCuRays, "a tapered launch has more rays");
-// ... and the smallest of those in units of 4 rays, which wait less on each
-// other and reach more CUs (12 K rays: 150 us, 159 in units of 16; 49 K rays:
-// no difference, at four times the waves).
+// The smallest launches run in quads whatever their units, of 4 rays then, which wait
+// less on each other and reach more CUs (12 K rays: 150 us, 159 in units of 16; 49 K
+// rays: no difference, at four times the waves; 16,384 envs of one ray on a 512^3 room
+// grid 200 us, 261 with a lane each).
 constexpr uint32_t kQuadSmallRays = 1u << 14;
 __host__ __device__ constexpr uint32_t axis_stride(uint32_t depth) { return (1u << depth) + 2u; }
 constexpr uint32_t kPlaneHeader = 8;  // floats before the planes: scales, pad, offsets, pad
@@ -1910,14 +1939,26 @@ int plane_depth_wide(int32_t n_scenes, uint32_t D, size_t budget) {
 // kernel traced it (every other launch: trace_relaid_kernel alone).
 int launch_relaid_queued(RelaidParams P, hipStream_t stream, uint32_t* scratch_queue, navi_launch_info& info);
 
-// A small batch on trace_quad_kernel: one wave per unit, no work queue (and no
-// queue pair: launches on any streams, captured or not, share nothing).
-int launch_quad(RelaidParams P, hipStream_t stream, navi_launch_info& info) {
-    const uint32_t D = P.cell_depth;
-    const bool poses = P.local_dirs != nullptr;
+// Sets a launch's units for trace_quad_kernel; whether it is one for it (kQuad*Units, all
+// 16 rays a unit or, below kQuadSmallRays, 4). fast_scenes: every scene is known to take
+// the fast march.
+bool quads_pay(RelaidParams& P, bool fast_scenes) {
     P.quad_shift = P.n_rays <= kQuadSmallRays ? 2u : 4u;
     const uint32_t unit = 1u << P.quad_shift;
     P.env_units = P.tile_el ? P.rays_per_env >> P.quad_shift : (P.rays_per_env + unit - 1u) / unit;
+    const uint32_t units = P.n_envs * P.env_units;  // at most n_rays, which is at most 2^30
+    if (P.n_rays <= kQuadSmallRays) return true;
+    if (!fast_scenes || !(P.max_distance < kOutsideDomain)) return units < kQuadGeneralUnits;
+    if (P.tile_el && P.rays_per_env >= kQuadFineRays) return units < kQuadTiledUnits;
+    const bool full = P.n_rays >= 15ull * units && P.rays_per_env >= kQuadEnvRays;  // 15 of a unit's 16 rays and more
+    return units < (full ? kQuadFullUnits : kQuadSparseUnits);
+}
+
+// A small batch on trace_quad_kernel: one wave per unit (of quads_pay), no work queue (and
+// no queue pair: launches on any streams, captured or not, share nothing).
+int launch_quad(RelaidParams P, hipStream_t stream, navi_launch_info& info) {
+    const uint32_t D = P.cell_depth;
+    const bool poses = P.local_dirs != nullptr;
     P.div_units = make_fastdiv(P.env_units);
     const uint32_t blocks = P.n_envs * P.env_units;
     void (*kernel)(RelaidParams) = nullptr;
@@ -1936,12 +1977,13 @@ int launch_quad(RelaidParams P, hipStream_t stream, navi_launch_info& info) {
     return NAVI_OK;
 }
 
-int launch_relaid(RelaidParams P, hipStream_t stream, uint32_t* scratch_queue = nullptr) {
+int launch_relaid(RelaidParams P, hipStream_t stream, uint32_t* scratch_queue = nullptr, bool fast_scenes = false) {
     navi_launch_info info = {};
     info.n_rays = P.n_rays;
     P.small_tables = (static_cast<uint64_t>(P.n_scenes) << (3u * P.cell_depth + 3u)) < (1ull << 32) ? 1u : 0u;
     const uint64_t wide_min = g_wide_min_rays.load(std::memory_order_relaxed);
-    if (P.n_rays < (wide_min == kWideMinRays ? kQuadMaxRays : std::min<uint64_t>(wide_min, kFastMinRays))) {
+    if (quads_pay(P, fast_scenes) &&
+        (wide_min == kWideMinRays || P.n_rays < std::min<uint64_t>(wide_min, kFastMinRays))) {
         info.pair = -1;
         const int code = launch_quad(P, stream, info);
         g_last_launch = info;
@@ -2187,7 +2229,7 @@ extern "C" int navi_trace_relaid_ex(const navi_relaid_launch* L, void* stream) {
         P.n_leaves = L->n_leaves;
         P.sem_bits = 16u;
     }
-    return launch_relaid(P, static_cast<hipStream_t>(stream));
+    return launch_relaid(P, static_cast<hipStream_t>(stream), nullptr, (L->scene_hints & NAVI_SCENES_FAST) != 0u);
 }
 
 

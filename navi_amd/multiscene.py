@@ -63,7 +63,8 @@ def wide_plane_depth(n_scenes: int, table_depth: int) -> int:
     ``plane_depth_wide``): the deepest P in [max(4, D - 2), min(D + 2, 8)] whose planes
     and scene table fit ``WIDE_PLANE_LDS_BYTES``; 0 when none does (such launches take
     the 256-thread workgroups). Launches of fewer rays than ``navi_set_wide_min_rays``
-    (default 2^19), and at its default launches below 851,968 rays, do not run on it."""
+    (default 2^19), and at its default those that run with four lanes per ray (up to
+    851,968 rays), do not run on it."""
     for p in range(min(table_depth + 2, 8), max(4, table_depth - 2) - 1, -1):
         if n_scenes * (32 + _plane_bytes(p)) <= WIDE_PLANE_LDS_BYTES:
             return p
@@ -229,6 +230,8 @@ class ResidentScenes:
             # 32-bit byte size must not wrap: fewer than 2^27 records
             if offset >= (1 << 27):
                 return False
+        fast = (rtable["flags"] & _native.SCENE_NONNEG_LEAVES).all() and (rtable["max_depth"] <= 30).all()
+        self._scene_hints = _native.SCENES_FAST if fast else 0
         self.n_records = offset
         self.record_counts = [int(c) for c in rtable["n_records"]]
         if n_leaves:
@@ -519,6 +522,7 @@ class ResidentScenes:
         if self.n_leaves:
             L.leaves, L.n_leaves = self.leaves.data_ptr(), self.n_leaves
         L.scenes, L.n_scenes = self.relaid_table.data_ptr(), self.n_scenes
+        L.scene_hints = self._scene_hints
         L.cell_tables, L.table_depth = self.cell_tables.data_ptr(), self.table_depth
         L.env_scene = env_scene_ptr
         L.env_order = order.data_ptr() if order is not None else None

@@ -83,3 +83,47 @@ def test_launch_shapes_of_mid_size_batches(resident, corpus, envs):  # noqa: F81
     # 256 CUs of 16 or 32 waves
     assert info["quad"] == (envs < 104) and (info["quad"] or info["waves"] == (4096 if envs < 160 else 8192)), info
     _compare(got, ref, 30.0, str(envs))
+
+
+# (envs, az, el, elevation_bins, max_distance, quads): units on both sides of each line. Envs of
+# 3 rays (a unit each), full units of 128 rays an env (8 each), in tiles too, of 127 (one idle
+# lane in 128, but an env too small for its neighbours to be alike), of 64 in tiles and of 16 (full,
+# too small); angular tiles over a general range (4 units each); 16,384 envs of one ray (the
+# smallest launches) and one more
+LINES = [(8191, 3, 1, 0, 30.0, True), (8192, 3, 1, 0, 30.0, False), (4095, 128, 1, 0, 30.0, True),
+         (4096, 128, 1, 0, 30.0, False), (1023, 127, 1, 0, 30.0, True), (1024, 127, 1, 0, 30.0, False),
+         (4095, 16, 8, 8, 30.0, True), (4096, 16, 8, 8, 30.0, False), (2047, 8, 8, 8, 30.0, True),
+         (2048, 8, 8, 8, 30.0, False), (8191, 16, 1, 0, 30.0, True), (8192, 16, 1, 0, 30.0, False), (1023, 8, 8, 8, 1200.0, True),
+         (1024, 8, 8, 8, 1200.0, False), (16384, 1, 1, 0, 30.0, True), (16385, 1, 1, 0, 30.0, False)]
+
+
+@pytest.mark.parametrize("envs,az,el,bins,max_distance,quads", LINES)
+def test_launches_of_many_units_leave_the_quads(resident, corpus, envs, az, el, bins, max_distance, quads):  # noqa: F811
+    from navi_amd import _native
+
+    env_scene, o, d = _rays(corpus, envs, az, el, seed=envs + az)
+    ref = _oracle_multi([c.words for c in corpus], [c.bbox_min_list + c.bbox_max for c in corpus],
+                        env_scene, o, d, 96, max_distance)
+    got = _run(resident, env_scene, o, d, 96, max_distance, elevation_bins=bins)
+    info = _native.last_launch()
+    assert info["quad"] == quads, info
+    _compare(got, ref, max_distance, f"{envs}x{az}x{el}/{bins}/{max_distance}")
+
+
+@pytest.mark.parametrize("envs,quads", [(1023, True), (1024, False)])
+def test_launches_of_negative_leaves_leave_the_quads_early(gpu, corpus, envs, quads):  # noqa: F811
+    """Scenes that need the general march: known to ResidentScenes, so their line is its."""
+    from navi_amd import _native
+    from navi_amd.multiscene import ResidentScenes
+
+    words = corpus[1].words.copy()
+    leaf = np.flatnonzero(words >> np.uint64(63))
+    words[leaf[leaf.size // 2]] |= np.uint64(0x8000)
+    bounds = corpus[1].bbox_min_list + corpus[1].bbox_max
+    resident = ResidentScenes([(words, bounds[:3], bounds[3:])])
+    env_scene, o, d = _rays(corpus[1:2], envs, 8, 8, seed=envs)
+    ref = _oracle_multi([words], [bounds], env_scene, o, d, 96, 30.0)
+    got = _run(resident, env_scene, o, d, 96, 30.0, elevation_bins=8)
+    info = _native.last_launch()
+    assert info["quad"] == quads, info
+    _compare(got, ref, 30.0, str(envs))
