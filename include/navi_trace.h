@@ -355,7 +355,8 @@ int navi_trace_relaid_poses(const uint32_t* records, uint64_t n_records, const n
 
 /* navi_relaid_launch.scene_hints: what the caller knows of the scene table, for
  * the launch shape (results are the same with or without). */
-#define NAVI_SCENES_FAST 1u /* every scene has NAVI_SCENE_NONNEG_LEAVES and max_depth <= 30 */
+#define NAVI_SCENES_FAST 1u /* every scene has NAVI_SCENE_NONNEG_LEAVES, max_depth <= 30 and a
+                               box at most 64 of its sides from the origin */
 
 /* Arguments of navi_trace_relaid_ex (device pointers unless noted). */
 typedef struct navi_relaid_launch {

@@ -470,10 +470,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) void tr
     const navi_relaid_scene& S = P.scenes[sc];
 
     // ---- what the fast march needs of the scene (see stage_scenes and
-    // stage_planes). With |off| <= 2^14 every plane lies within 2^-6 cell of
+    // stage_planes). With |off| <= 2^16 every plane lies within 2^-5 cell of
     // the uniform grid: a level's midpoint is off by at most half an ulp of the
-    // largest coordinate, which is below (2^14 + 2^8) cells, and eight levels
-    // add up to 2^-21 of it. ----
+    // largest coordinate, 2^-24 of (2^16 + 2^8) cells, which eight levels add
+    // up, and the offset is exact to half of its ulp, 2^-8 cell: what plane_cell
+    // allows is 0.2 cell and more. (The combined kernel's planes are 2^6, so its
+    // 2^14 reaches as far: a 512^3 room grid 100 of its sides from the origin,
+    // 49 K rays, takes 209 us, 324 in the general march.) ----
     const float lo_a = S.bbox_min[ax], hi_a = S.bbox_max[ax];
     const float extent = hi_a - lo_a;
     const float scale = static_cast<float>(kCells) / extent;
@@ -481,7 +484,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) void tr
     const double cw = (static_cast<double>(hi_a) - static_cast<double>(lo_a)) / kCells;
     const bool axis_ok = fabsf(lo_a) < 0x1p100f && fabsf(hi_a) < 0x1p100f && extent > 0.0f && scale > 0.0f &&
                          scale <= 0x1p127f && cw > 0.0 && fabs(static_cast<double>(scale) * cw - 1.0) <= 1e-6 &&
-                         fabsf(off) <= 0x1p14f;
+                         fabsf(off) <= 0x1p16f;
     const bool shallow = S.max_depth <= static_cast<uint32_t>(kMaxDepth - 2);
     const bool monotone = (S.flags & NAVI_SCENE_NONNEG_LEAVES) != 0u;
     const bool fast = shallow && monotone && P.small_tables != 0u && P.max_distance < kOutsideDomain &&

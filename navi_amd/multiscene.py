@@ -230,7 +230,9 @@ class ResidentScenes:
             # 32-bit byte size must not wrap: fewer than 2^27 records
             if offset >= (1 << 27):
                 return False
-        fast = (rtable["flags"] & _native.SCENE_NONNEG_LEAVES).all() and (rtable["max_depth"] <= 30).all()
+        lo, hi = rtable["bbox_min"].astype(np.float64), rtable["bbox_max"].astype(np.float64)
+        fast = ((rtable["flags"] & _native.SCENE_NONNEG_LEAVES).all() and (rtable["max_depth"] <= 30).all()
+                and (np.abs(lo) <= 64 * (hi - lo)).all())
         self._scene_hints = _native.SCENES_FAST if fast else 0
         self.n_records = offset
         self.record_counts = [int(c) for c in rtable["n_records"]]

@@ -127,3 +127,27 @@ def test_launches_of_negative_leaves_leave_the_quads_early(gpu, corpus, envs, qu
     info = _native.last_launch()
     assert info["quad"] == quads, info
     _compare(got, ref, 30.0, str(envs))
+
+
+@pytest.mark.parametrize("sides", [0, 30, 60, 100, 200, 254, 258, 1000])
+def test_scenes_far_from_the_origin(gpu, corpus, sides):  # noqa: F811
+    """Boxes up to 256 of their sides away take the quads' fast march (off <= 2^16), farther
+    ones the general march; depth-8 cells are 2^8 ulps wide at that line."""
+    from navi_amd import _native
+    from navi_amd.multiscene import ResidentScenes
+
+    scene = corpus[1]
+    lo, hi = np.float32(scene.bbox_min_list), np.float32(scene.bbox_max)
+    side = hi[0] - lo[0]
+    shift = np.float32([sides, -sides, sides]) * side
+    lo, hi = lo + shift, hi + shift
+    resident = ResidentScenes([(scene.words, lo.tolist(), hi.tolist())])
+    env_scene, o, d = _rays(corpus[1:2], 6, 32, 16, seed=sides + 1)
+    rng = np.random.default_rng(sides)
+    o = (o + shift).astype(np.float32)
+    o[3:] = rng.uniform(lo, hi, o[3:].shape)  # any place, cell faces among them at this spacing
+    ref = _oracle_multi([scene.words], [lo.tolist() + hi.tolist()], env_scene, o, d, 160, 30.0)
+    got = _run(resident, env_scene, o, d, 160, 30.0, elevation_bins=16)
+    assert _native.last_launch()["quad"]
+    assert resident._scene_hints == (_native.SCENES_FAST if sides <= 60 else 0)
+    _compare(got, ref, 30.0, f"{sides} sides away")
