@@ -63,6 +63,19 @@ def test_chunked_envs_match_the_oracle(gpu, corpus, e, az, el):  # noqa: F811
         assert np.array_equal(part[1].view(np.uint32), got[1].view(np.uint32))
 
 
+# envs that end below, at and past a wave's run: of 64 elements (El not in fours), of 256 (16-byte
+# accesses), of a round of all 512 or 1024 threads
+ENDS = [(9, 7), (32, 2), (13, 5), (63, 4), (64, 4), (65, 4), (73, 7), (128, 4), (171, 3), (1023, 4), (1024, 4),
+        (1025, 4), (24, 9)]
+
+
+@pytest.mark.parametrize("e", [2, 258])
+@pytest.mark.parametrize("az,el", ENDS)
+def test_small_envs_match_the_oracle(gpu, corpus, e, az, el):  # noqa: F811
+    """Waves that hold none of their env's elements leave the round early."""
+    test_chunked_envs_match_the_oracle(gpu, corpus, e, az, el)
+
+
 @pytest.mark.parametrize("e", [6, 262])
 def test_first_frame_is_decided_by_the_whole_row(gpu, corpus, e):  # noqa: F811
     """The delta is zero exactly where |previous depth| sums below 1e-6: rows of zeros, of
