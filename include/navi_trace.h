@@ -398,15 +398,15 @@ int navi_trace_relaid_ex(const navi_relaid_launch* launch, void* stream);
 
 /*
  * Launch shape of the record-layout tracer (no reference counterpart: a tuning
- * knob of this library). Launches of at least `n_rays` rays whose scenes'
- * split planes fit two levels below the cell tables in 80 KiB of LDS run in
- * 1024-thread workgroups, a lane per ray; smaller launches below 2^19 rays that
- * suit it run with four lanes per ray (trace_quad_kernel), others in 256-thread
- * workgroups. At the default threshold launches of up to 851,968 rays that suit it
- * (a fine sensor's angular tiles; fewer in other orders, in envs of few rays,
- * without NAVI_SCENES_FAST or over 1000 m) run with four lanes per ray. Results are
- * identical either way. Process-wide, thread-safe; takes effect from the next
- * launch. Returns the previous value (default 2^19).
+ * knob of this library). At the default, launches of up to 851,968 rays that suit
+ * it (a fine sensor's angular tiles; fewer in other orders, in envs of few rays,
+ * without NAVI_SCENES_FAST or over 1000 m) run with four lanes per ray
+ * (trace_quad_kernel). Of the others, and of all launches at another value, those
+ * of at least `n_rays` rays whose scenes' split planes fit two levels below the
+ * cell tables in 80 KiB of LDS run in 1024-thread workgroups, a lane per ray,
+ * the rest in 256-thread ones. Results are identical either way. Process-wide,
+ * thread-safe; takes effect from the next launch. Returns the previous value
+ * (default 2^19).
  */
 uint64_t navi_set_wide_min_rays(uint64_t n_rays);
 

@@ -326,8 +326,9 @@ def lib() -> ctypes.CDLL:
 
 def set_wide_min_rays(n_rays: int) -> int:
     """Launches of the record-layout tracer with at least ``n_rays`` rays run in
-    1024-thread workgroups when their split planes fit (results are identical);
-    returns the previous threshold."""
+    1024-thread workgroups when their split planes fit, and at another value than the
+    default none run with four lanes per ray (results are identical); returns the previous
+    threshold."""
     if not 0 <= int(n_rays) < (1 << 64):
         raise ValueError("n_rays must fit an unsigned 64-bit integer")
     return int(_lib.navi_set_wide_min_rays(int(n_rays)))

@@ -49,7 +49,6 @@
 // multiply-high division by the (uniform) rays-per-env and tile counts.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <map>
@@ -293,14 +292,14 @@ constexpr size_t kFastLds = 20480;
 constexpr int kWideThreads = 1024;
 constexpr size_t kFastLdsWide = 81920;
 // Launches of at least so many rays run wide where trace_quad_kernel does not take
-// them; with the threshold raised (navi_set_wide_min_rays), launches
-// below it take the 256-thread workgroups from kFastMinRays rays on, which spread
-// a batch over more CUs (786 K rays on one 512^3 scene 3% faster wide).
+// them. With the threshold moved (navi_set_wide_min_rays) none is taken by it: smaller
+// launches run in 256-thread workgroups, from kFastMinRays rays on with the fast kernel
+// first, which spread a batch over more CUs (786 K rays on one 512^3 scene 3% faster wide).
 constexpr uint64_t kWideMinRays = 1u << 19;
 std::atomic<uint64_t> g_wide_min_rays{kWideMinRays};
-// Launches of fewer rays skip the 256-thread fast kernel (a lowered wide
-// threshold whose planes do not fit): the combined kernel alone saves the
-// second launch.
+// Launches of fewer rays skip the 256-thread fast kernel: the combined kernel alone saves
+// the second launch. (Only a raised wide threshold reaches that kernel: where its planes
+// fit, the wide shape's do.)
 constexpr uint32_t kFastMinRays = 1u << 19;
 // Launches of few units (of 16 rays, or 4) take trace_quad_kernel, four lanes per ray:
 // they last as long as their longest rays' chains of steps, and a quad's step takes about
@@ -1982,8 +1981,7 @@ int launch_relaid(RelaidParams P, hipStream_t stream, uint32_t* scratch_queue = 
     info.n_rays = P.n_rays;
     P.small_tables = (static_cast<uint64_t>(P.n_scenes) << (3u * P.cell_depth + 3u)) < (1ull << 32) ? 1u : 0u;
     const uint64_t wide_min = g_wide_min_rays.load(std::memory_order_relaxed);
-    if (quads_pay(P, fast_scenes) &&
-        (wide_min == kWideMinRays || P.n_rays < std::min<uint64_t>(wide_min, kFastMinRays))) {
+    if (wide_min == kWideMinRays && quads_pay(P, fast_scenes)) {
         info.pair = -1;
         const int code = launch_quad(P, stream, info);
         g_last_launch = info;

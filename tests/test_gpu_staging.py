@@ -7,7 +7,7 @@ fast march's launches), for 8x8 tiles and for linear ray order, explicit rays an
 rays from poses, env orders with skipped entries, unknown scene ids, a batch with
 many tiles per wave (slots evicted while rays of their tile still march) and the
 no-allocation entry point; one staged launch is checked against the oracle too. Every
-test runs in both launch shapes (256- and 1024-thread workgroups).
+test runs in both launch shapes with a lane per ray (256- and 1024-thread workgroups).
 """
 
 from __future__ import annotations
@@ -31,16 +31,15 @@ def _say(msg: str) -> None:
 
 @pytest.fixture(scope="module", params=["wg256", "wg1024"])
 def pool(gpu, request):
-    """The scene pool; the module runs twice: the default launch shape for these
-    small batches (256-thread workgroups, planes above the tables) and the wide one
-    (1024-thread workgroups, planes two levels below the tables), forced through
-    navi_set_wide_min_rays."""
+    """The scene pool; the module runs twice: in 256-thread workgroups (planes above the
+    tables) and in the wide shape (1024-thread workgroups, planes two levels below the
+    tables), both forced through navi_set_wide_min_rays."""
     import torch
 
     from navi_amd import _native
     from navi_amd import scenes as S
 
-    prev = _native.set_wide_min_rays(0 if request.param == "wg1024" else 1 << 19)
+    prev = _native.set_wide_min_rays(0 if request.param == "wg1024" else (1 << 64) - 1)
     request.addfinalizer(lambda: _native.set_wide_min_rays(prev))
 
     scenes = [S.rooms(seed=3, resolution=128), S.cluttered(seed=2, resolution=128), S.box_room(seed=4, resolution=64)]
@@ -67,7 +66,7 @@ def pool(gpu, request):
     dev = torch.device("cuda:0")
     _native.device_init(dev)
     return {
-        "scenes": scenes, "n_records": allrec.shape[0], "dev": dev,
+        "wide": request.param == "wg1024", "scenes": scenes, "n_records": allrec.shape[0], "dev": dev,
         "records": torch.from_numpy(allrec.view(np.int32).reshape(-1).copy()).to(dev),
         "table": torch.from_numpy(rtable.view(np.uint8).copy()).to(dev),
         "cells": torch.from_numpy(tables.view(np.int64)).to(dev),
@@ -112,6 +111,10 @@ def _launch(pool, name, env_scene, env_order, E, R, el, a, b, c=None, steps=Fals
     else:
         args = head + (a.data_ptr(), b.data_ptr()) + tail
     _native.check(getattr(lib, name)(*args))
+    info = _native.last_launch()
+    assert not info["quad"] and info["fast_wide"] == pool["wide"] and info["staged"] != steps, info
+    assert info["queue"] == ("scratch" if name == "navi_trace_relaid_noalloc" else "stream"), info
+    assert info["fast"] == (pool["wide"] or E * R >= 1 << 19), info
     torch.cuda.synchronize()
     return od.cpu().numpy(), os_.cpu().numpy(), (on.cpu().numpy() if steps else None)
 

@@ -8,6 +8,9 @@ work-queue counters live in a static device array), called through the C ABI:
 * the outputs of those two calls equal navi_trace_relaid's on the same inputs:
   distances, semantics and step counts bit for bit.
 
+Both with four lanes per ray, which needs no counters, and with a lane per ray in either
+launch shape, which does.
+
 The scene pool is built here without ResidentScenes; in a fresh process the warm-up
 call is also the entry point's first call on the device (no navi_device_init before
 it), while in a full test run earlier tests have initialised the device already.
@@ -51,6 +54,21 @@ def _pool(scenes, depth):
 
 
 def test_noalloc_allocates_nothing_and_matches_navi_trace_relaid(gpu):
+    _check_noalloc({"quad": True, "fast_wide": False, "queue": "none"})
+
+
+@pytest.mark.parametrize("wide", [False, True])
+def test_noalloc_with_a_lane_per_ray(gpu, wide):
+    from navi_amd import _native
+
+    prev = _native.set_wide_min_rays(0 if wide else (1 << 64) - 1)
+    try:
+        _check_noalloc({"quad": False, "fast_wide": wide, "queue": "scratch"})
+    finally:
+        _native.set_wide_min_rays(prev)
+
+
+def _check_noalloc(shape):
     import torch
 
     from navi_amd import _native
@@ -94,6 +112,9 @@ def test_noalloc_allocates_nothing_and_matches_navi_trace_relaid(gpu):
             c["es"].data_ptr(), None, c["E"], c["R"], c["el"], c["o"].data_ptr(), c["d"].data_ptr(),
             od.data_ptr(), os_.data_ptr(), 128, 30.0, 0.01, on.data_ptr(), stream)
         _native.check(code)
+        info = _native.last_launch()
+        queue = "stream" if name == "navi_trace_relaid" and not shape["quad"] else shape["queue"]
+        assert {k: info[k] for k in shape} == dict(shape, queue=queue), info
 
     call("navi_trace_relaid_noalloc", 1)  # warm-up: the runtime loads the kernels on first launch
     torch.cuda.synchronize()
