@@ -70,10 +70,10 @@ typedef struct navi_launch_info {
  * no record deeper than 30 levels; the device checks the scene table) and
  * otherwise hands the launch to trace_relaid_kernel, enqueued after it. */
 #define NAVI_KERNEL_FAST 1u         /* trace_fast_kernel */
-#define NAVI_KERNEL_FAST_WIDE 2u    /* ... in 1024-thread workgroups (two per CU) */
+#define NAVI_KERNEL_FAST_WIDE 2u    /* ... in 1024-thread workgroups (one or two per CU) */
 #define NAVI_KERNEL_COMBINED 4u     /* trace_relaid_kernel (both marches, seven waves per SIMD) */
 #define NAVI_KERNEL_RAW 8u          /* the word-layout kernel (navi_cast_rays, navi_cast_rays_multi) */
-#define NAVI_KERNEL_QUAD 16u        /* with COMBINED: trace_quad_kernel instead (both marches, four lanes per ray) */
+#define NAVI_KERNEL_QUAD 16u        /* trace_quad_kernel alone (both marches, four lanes per ray) */
 /* navi_launch_info.queue */
 #define NAVI_QUEUE_NONE 0u     /* no pair: trace_quad_kernel, which needs none, or a static schedule
                                   without trace_fast_kernel */

@@ -1967,7 +1967,7 @@ int launch_quad(RelaidParams P, hipStream_t stream, navi_launch_info& info) {
         case 6: kernel = poses ? trace_quad_kernel<6, true> : trace_quad_kernel<6, false>; break;
         default: kernel = poses ? trace_quad_kernel<7, true> : trace_quad_kernel<7, false>; break;
     }
-    info.kernels = NAVI_KERNEL_COMBINED | NAVI_KERNEL_QUAD;
+    info.kernels = NAVI_KERNEL_QUAD;
     info.planes = kQuadPlanes;
     info.waves = blocks;
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64), 0, stream, P);

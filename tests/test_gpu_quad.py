@@ -41,6 +41,7 @@ def test_quad_units_match_the_oracle(resident, corpus, envs, az, el, bins, max_d
     got = _run(resident, env_scene, o, d, 160, max_distance, elevation_bins=bins)
     info = _native.last_launch()
     assert info["quad"] and info["n_rays"] == envs * az * el, info
+    assert not (info["combined"] or info["fast"] or info["raw"]), info  # nothing else is enqueued
     _compare(got, ref, max_distance, f"{envs}x{az}x{el}/{bins}/{max_distance}")
 
 

@@ -47,6 +47,22 @@ def wide_for_every_launch():
         _native.set_wide_min_rays(old)
 
 
+@contextlib.contextmanager
+def launch_shape(shape):
+    """"quads": the default, four lanes per ray for small batches; "combined": the combined
+    kernel alone for them; "wide": the 1024-thread fast kernel first."""
+    from navi_amd import _native
+
+    old = _native.set_wide_min_rays({"quads": 1 << 19, "combined": (1 << 64) - 1, "wide": 0}[shape])
+    try:
+        yield
+    finally:
+        _native.set_wide_min_rays(old)
+
+
+SHAPES = ("quads", "combined", "wide")
+
+
 @pytest.fixture(scope="module")
 def scenes():
     from navi_amd import scenes as S
@@ -303,16 +319,18 @@ def test_wide_semantics_on_the_record_layout(gpu, scenes):
         out_s = torch.empty((E, R), device=dev, dtype=torch.int32)
         out_n = torch.empty((E, R), device=dev, dtype=torch.int32)
         for with_steps in (False, True):
-            for wide_shape in (False, True):  # the combined kernel alone, or the 1024-thread fast kernel first
-                with wide_for_every_launch() if wide_shape else contextlib.nullcontext():
+            for shape in SHAPES:
+                with launch_shape(shape):
                     out_d.fill_(float("nan"))
                     out_s.fill_(-7)
                     res.cast_rays(es, o, d, out_d, out_s, 128, 30.0, elevation_bins=el,
                                   out_steps=out_n if with_steps else None)
                 info = _native.last_launch()
-                assert not info["raw"] and info["combined"] and info["fast_wide"] == wide_shape, info
+                assert {k: info[k] for k in ("raw", "quad", "combined", "fast_wide")} == {
+                    "raw": False, "quad": shape == "quads", "combined": shape != "quads",
+                    "fast_wide": shape == "wide"}, info
                 torch.cuda.synchronize()
-                _check(out_d, out_s, ref, f"scenes {launch_scenes}, steps {with_steps}, wide {wide_shape}")
+                _check(out_d, out_s, ref, f"scenes {launch_scenes}, steps {with_steps}, {shape}")
                 if with_steps:
                     assert np.array_equal(out_n.cpu().numpy(), ref["steps"])
         # rays from poses: the same rays, built in the kernel
@@ -323,12 +341,12 @@ def test_wide_semantics_on_the_record_layout(gpu, scenes):
         pd[..., 1] = local[None, :, 1]
         pd[..., 2] = (-local[None, :, 0]) * s_ + local[None, :, 2] * c
         pref = oracle.trace_multi(pool, base, nw, bounds, env_scene, origins, pd, 128, 30.0, threads=_threads())
-        for wide_shape in (False, True):
-            with wide_for_every_launch() if wide_shape else contextlib.nullcontext():
+        for shape in SHAPES:
+            with launch_shape(shape):
                 res.cast_rays_poses(es, torch.from_numpy(local).to(dev), torch.from_numpy(origins_env).to(dev), rot,
                                     out_d, out_s, 128, 30.0, elevation_bins=el)
             torch.cuda.synchronize()
-            _check(out_d, out_s, pref, f"poses, scenes {launch_scenes}, wide {wide_shape}")
+            _check(out_d, out_s, pref, f"poses, scenes {launch_scenes}, {shape}")
     # point queries in every scene
     pts = np.concatenate([rng.uniform(s.bbox_min_list, s.bbox_max, (300, 3)) for s in sc_of]).astype(np.float32)
     pscene = np.repeat(np.arange(3, dtype=np.int32), 300)
