@@ -7,6 +7,7 @@ each against the oracle or an eager launch bit for bit:
   runs after more captures than the table holds;
 * reserve pairs leased per launch once every table pair is taken (one raw HIP
   stream per launch);
+* launches captured while no pair is left, on the static schedule;
 * leaves of semantic 0x7fff and above traced on the record layout (fast and general
   march, rays from poses, point queries, the drop-in).
 """
@@ -259,6 +260,72 @@ def test_leased_pairs_when_the_table_is_full(setup):
             assert len(set(leases)) >= 1
     finally:
         torch.cuda.synchronize()
+        for s in streams:
+            hip.hipStreamDestroy(s)
+
+
+@pytest.mark.parametrize("shape", ["combined", "wide"])
+@pytest.mark.parametrize("with_steps", [False, True])
+def test_static_schedule_when_no_pair_is_left(setup, shape, with_steps):
+    """With the table's pairs taken by streams and by graphs that are alive, a captured launch
+    gets no counters: trace_relaid_kernel alone, every wave its own share of the rays. The
+    graph's replays give the oracle's results."""
+    import torch
+
+    from navi_amd import _native
+
+    t = setup
+    res, E, R = t["res"], t["E"], t["R"]
+    dev = res.device
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    hip.hipStreamCreate.argtypes = [ctypes.POINTER(ctypes.c_void_p)]
+    hip.hipStreamDestroy.argtypes = [ctypes.c_void_p]
+    out_d = torch.empty((E, R), device=dev)
+    out_s = torch.empty((E, R), device=dev, dtype=torch.int32)
+    out_n = torch.empty((E, R), device=dev, dtype=torch.int32) if with_steps else None
+    streams, graphs = [], []
+    cap = torch.cuda.Stream()
+
+    def launch():
+        res.cast_rays(t["es"], t["o"], t["d"], out_d, out_s, 128, 30.0, out_steps=out_n, elevation_bins=t["el"])
+
+    try:
+        with launch_shape(shape):
+            for _ in range(2):
+                launch()
+                torch.cuda.synchronize()
+            while len(streams) < 4200:
+                s = ctypes.c_void_p()
+                assert hip.hipStreamCreate(ctypes.byref(s)) == 0
+                streams.append(s)
+                with torch.cuda.stream(torch.cuda.ExternalStream(s.value)):
+                    launch()
+                if _native.last_launch()["queue"] == "lease":
+                    break
+            torch.cuda.synchronize()
+            while len(graphs) < 4200:
+                graphs.append(torch.cuda.CUDAGraph())
+                with torch.cuda.graph(graphs[-1], stream=cap):
+                    launch()
+                info = _native.last_launch()
+                if info["queue"] != "capture":
+                    break
+        assert info["queue"] == "none" and info["combined"] and not info["fast"] and not info["quad"], info
+        _say(f"{shape}, steps {with_steps}: {len(streams)} streams, {len(graphs)} graphs")
+        for rep in range(3):
+            out_d.fill_(float("nan"))
+            out_s.fill_(-7)
+            torch.cuda.synchronize()
+            graphs[-1].replay()
+            torch.cuda.synchronize()
+            _check(out_d, out_s, t["ref"], f"replay {rep}")
+            if with_steps:
+                assert np.array_equal(out_n.cpu().numpy(), t["ref"]["steps"])
+                out_n.fill_(-7)
+    finally:
+        torch.cuda.synchronize()
+        graphs.clear()
+        gc.collect()
         for s in streams:
             hip.hipStreamDestroy(s)
 
