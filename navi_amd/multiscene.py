@@ -244,8 +244,9 @@ class ResidentScenes:
             allrec = np.concatenate(recs) if offset else np.zeros(8, np.uint32)
             self.records = torch.from_numpy(allrec.view(np.int32)).to(self.device)
         else:
-            self.records = torch.cat([r if isinstance(r, torch.Tensor) else
-                                      torch.from_numpy(r.view(np.int32)).to(self.device) for r in recs])
+            recs = [r if isinstance(r, torch.Tensor) else torch.from_numpy(r.view(np.int32)).to(self.device)
+                    for r in recs]
+            self.records = torch.cat(recs) if len(recs) > 1 else recs[0]
         cells = 8 ** self.table_depth
         roots = [int(r) for r in rtable["root_slot"]]
         if self.device.type == "cuda":
