@@ -23,10 +23,11 @@
 //
 // What bounds it: the chain of one step, about 1400 cycles of which half are
 // its four to five dependent reads (a cell table one level deeper saves one
-// and 60 ns a step) and half its ~75 vector and ~90 scalar instructions, which
-// a lone wave issues one every four to five cycles. 47 VGPRs, eight waves per
-// SIMD. 1024 rays of a 64^3 room: 53 -> 36 us; 49 K rays of a 128^3 volume:
-// 112 -> 72 us; 49 K rays of a 1024^3 volume: 209 -> 140 us. A per-ray cache of
+// and 60 ns a step) and half its instructions (up to about 100 vector and 90
+// scalar ones), which a lone wave issues one every four to five cycles. 43
+// VGPRs, eight waves per SIMD. A pass with a lane per ray and with four: 1024 rays
+// of a 64^3 room 48 and 32 us; 49 K rays of a 128^3 volume 120 and 68; 49 K rays of
+// a 1024^3 volume with their observation 263 and 152. A per-ray cache of
 // the last depth-8 cell's slot made no difference: a wave skips the reads only
 // when all its rays hit.
 #pragma once

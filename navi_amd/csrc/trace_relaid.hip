@@ -325,12 +325,12 @@ constexpr uint32_t kQuadFineRays = 2048;  // rays of such a sensor
 //   409, 196 and 354.
 constexpr uint32_t kQuadFullUnits = 1u << 15;
 // * units with idle lanes, and those of so few rays an env that neighbours have little in
-//   common: 8192 units, as many as the chip holds at once.
-//   Rays in random directions, quads and a lane each: 65 K rays of 1, 2, 8 and 17 an env
-//   (65,536, 32,768, 8192 and 7710 units) on a 512^3 room grid 469, 356, 212 and 243 us
-//   against 282, 281, 273 and 274; 131 K of 8, 17 and 33 an env (16,384, 15,420 and 11,916
-//   units) 330, 363 and 279 against 300, 293 and 290; 262 K of 48 an env (16,384 full units)
-//   392 against 367; 800 K of one an env 4360 against 714.
+//   common: 8192 units, as many as the chip holds at once. Rays in random directions, quads
+//   and a lane each: 65 K rays of 1, 2, 8 and 17 an env (65,536, 32,768, 8192 and 7710 units)
+//   on a 512^3 room grid 469, 356, 212 and 243 us against 282, 281, 273 and 274; 131 K of 8, 17
+//   and 33 an env (16,384, 15,420 and 11,916 units) 330, 363 and 279 against 300, 293 and 290;
+//   262 K of 48 an env (16,384 full units) 392 against 367; 800 K of one an env 4360 against
+//   714 (547 in one workgroup per CU).
 constexpr uint32_t kQuadSparseUnits = 1u << 13;
 constexpr uint32_t kQuadEnvRays = 128;
 // * launches of the general march, whose step in quads is longer (ranges of 1000 and more,
