@@ -159,7 +159,11 @@ class ResidentScenes:
         # device record layout (one 32-byte record per internal node)
         self.n_leaves = 0
         self.leaves = None
-        self.relaid_ok = self._layout(chunks, table_depth)
+        if self.device.type == "cuda":
+            with torch.cuda.device(self.device):
+                self.relaid_ok = self._layout(chunks, table_depth, torch.cuda.current_stream(self.device))
+        else:
+            self.relaid_ok = self._layout(chunks, table_depth, None)
         self._order_key = None
         self._order = None
         # scene order by measured cost (module docstring)
@@ -203,12 +207,15 @@ class ResidentScenes:
         deepest = max(int(d) for d in rtable["max_depth"])  # 0xffffffff for a cycle
         return max(4, min(default_table_depth(self.n_scenes), deepest + 1))
 
-    def _layout(self, chunks: list, table_depth: int | None) -> bool:
+    def _layout(self, chunks: list, table_depth: int | None, stream: Any) -> bool:
         """The record layout of the scenes: records (child records as pool indices), cell
-        tables, leaf table, scene table. Each scene's records are converted on the device,
-        or on the host where the device does not cover it; both give the same arrays. False
-        when the record layout cannot hold the scenes. Waits for the device: the arrays are
-        complete for every stream when it returns."""
+        tables, leaf table, scene table. Each scene's records are converted on the device
+        (the current one, on ``stream``), or on the host where the device does not cover it;
+        both give the same arrays. False when the record layout cannot hold the scenes. Waits
+        for the device: the arrays are complete for every stream when it returns."""
+        state = None
+        if stream is not None:
+            state = torch.empty(_native.RELAYOUT_STATE_WORDS, dtype=torch.int32, device=self.device)
         rtable = np.zeros(self.n_scenes, dtype=_native.RELAID_SCENE_DTYPE)
         rtable["bbox_min"] = self.host_table["bbox_min"]
         rtable["bbox_max"] = self.host_table["bbox_max"]
@@ -216,7 +223,7 @@ class ResidentScenes:
         leaf_tables = []
         offset = n_leaves = 0
         for i, chunk in enumerate(chunks):
-            converted = (self._layout_on_device(rtable[i], i, chunk, offset)
+            converted = (self._layout_on_device(rtable[i], i, chunk, offset, state, stream)
                          or self._layout_on_host(rtable[i], chunk, offset, n_leaves))
             if not converted:
                 return False
@@ -230,9 +237,9 @@ class ResidentScenes:
             # 32-bit byte size must not wrap: fewer than 2^27 records
             if offset >= (1 << 27):
                 return False
-        lo, hi = rtable["bbox_min"].astype(np.float64), rtable["bbox_max"].astype(np.float64)
-        fast = ((rtable["flags"] & _native.SCENE_NONNEG_LEAVES).all() and (rtable["max_depth"] <= 30).all()
-                and (np.abs(lo) <= 64 * (hi - lo)).all())
+        fast = all(row["flags"] & _native.SCENE_NONNEG_LEAVES and row["max_depth"] <= 30
+                   and all(abs(a) <= 64 * (b - a) for a, b in zip(row["bbox_min"].tolist(), row["bbox_max"].tolist()))
+                   for row in rtable)
         self._scene_hints = _native.SCENES_FAST if fast else 0
         self.n_records = offset
         self.record_counts = [int(c) for c in rtable["n_records"]]
@@ -249,43 +256,43 @@ class ResidentScenes:
             self.records = torch.cat(recs) if len(recs) > 1 else recs[0]
         cells = 8 ** self.table_depth
         roots = [int(r) for r in rtable["root_slot"]]
-        if self.device.type == "cuda":
-            self.cell_tables = torch.empty(self.n_scenes * cells, dtype=torch.int64, device=self.device)
-            with torch.cuda.device(self.device):
-                current = torch.cuda.current_stream(self.device)
-                for i, root in enumerate(roots):
-                    _native.check(_native.lib().navi_build_cell_table_device(
-                        self.records.data_ptr(), self.n_records, root, self.table_depth,
-                        self.cell_tables.data_ptr() + 8 * cells * i, current.cuda_stream))
-                current.synchronize()
-        else:
+        if stream is None:
             tables = np.concatenate([_native.cell_table(allrec[:8 * offset], root, self.table_depth)
                                      for root in roots])
             self.cell_tables = torch.from_numpy(tables.view(np.int64))
+            self.relaid_table = torch.from_numpy(rtable.view(np.uint8).copy())
+            return True
+        self.cell_tables = torch.empty(self.n_scenes * cells, dtype=torch.int64, device=self.device)
+        for i, root in enumerate(roots):
+            _native.check(_native.lib().navi_build_cell_table_device(
+                self.records.data_ptr(), self.n_records, root, self.table_depth,
+                self.cell_tables.data_ptr() + 8 * cells * i, stream.cuda_stream))
+        # (the upload waits for the stream as well: one wait for both)
         self.relaid_table = torch.from_numpy(rtable.view(np.uint8).copy()).to(self.device)
+        stream.synchronize()
         return True
 
-    def _layout_on_device(self, entry: Any, i: int, chunk: Any, offset: int) -> tuple[Any, Any] | None:
+    def _layout_on_device(self, entry: Any, i: int, chunk: Any, offset: int, state: Any,
+                          stream: Any) -> tuple[Any, Any] | None:
         """Scene ``i``'s records, the pool's from ``offset`` on, converted on the device
-        (``navi_relayout_device``) and its ``entry`` of the scene table; None for a small
-        scene (``DEVICE_MIN_WORDS``) and when that leaves the scene to the host."""
-        if self.device.type != "cuda" or self.word_counts[i] < DEVICE_MIN_WORDS:
+        (``navi_relayout_device``) and its ``entry`` of the scene table; None without a
+        device, for a small scene (``DEVICE_MIN_WORDS``) and when that leaves the scene to
+        the host."""
+        n = self.word_counts[i]
+        if stream is None or n < DEVICE_MIN_WORDS:
             return None
-        lib = _native.lib()
-        with torch.cuda.device(self.device):
-            stream = torch.cuda.current_stream(self.device).cuda_stream
-            state = torch.empty(_native.RELAYOUT_STATE_WORDS, dtype=torch.int32, device=self.device)
-            n, at = self.word_counts[i], int(self.host_table[i]["word_offset"])
-            words = self.pool[at:at + n] if self.pool is not None else self._words(chunk).to(self.device)
-            mark, order = (torch.empty(n, dtype=torch.int32, device=self.device) for _ in range(2))
-            layout = _native.DeviceLayout()
-            _native.check(lib.navi_relayout_device(words.data_ptr(), n, mark.data_ptr(), order.data_ptr(),
-                                                   state.data_ptr(), ctypes.byref(layout), stream))
-            if not layout.converted:
-                return None
-            records = torch.empty(8 * layout.n_records, dtype=torch.int32, device=self.device)
-            _native.check(lib.navi_relayout_device_records(words.data_ptr(), n, mark.data_ptr(), order.data_ptr(),
-                                                           layout.n_records, offset, records.data_ptr(), stream))
+        lib, on = _native.lib(), stream.cuda_stream
+        at = int(self.host_table[i]["word_offset"])
+        words = self.pool[at:at + n] if self.pool is not None else self._words(chunk).to(self.device)
+        mark, order = (torch.empty(n, dtype=torch.int32, device=self.device) for _ in range(2))
+        layout = _native.DeviceLayout()
+        _native.check(lib.navi_relayout_device(words.data_ptr(), n, mark.data_ptr(), order.data_ptr(),
+                                               state.data_ptr(), ctypes.byref(layout), on))
+        if not layout.converted:
+            return None
+        records = torch.empty(8 * layout.n_records, dtype=torch.int32, device=self.device)
+        _native.check(lib.navi_relayout_device_records(words.data_ptr(), n, mark.data_ptr(), order.data_ptr(),
+                                                       layout.n_records, offset, records.data_ptr(), on))
         entry["rec_offset"] = entry["root_slot"] = offset
         entry["n_records"], entry["max_depth"], entry["flags"] = layout.n_records, layout.max_depth, layout.flags
         return records, None
